@@ -304,6 +304,9 @@ int pbe_copy_ops(const pbe_copy_op* ops, int64_t n_ops, int device, void* stream
  * outside the arena or not a page id, or whose length needs more than
  * max_blocks_per_seq blocks, gets NaN outputs (its pages are not read past
  * the failing id). splits = 0 picks pbe_paged_decode_splits(); at most 1024.
+ * `splits` sizes the partials: the batch's blocks are cut into pieces of about
+ * equal length, at most batch * splits of them (longer sequences take more
+ * than `splits`, shorter ones fewer); 1 leaves every sequence whole.
  * workspace: at least pbe_paged_decode_workspace_bytes() bytes of device
  * memory, used by this launch until it completes. Asynchronous on `stream`. */
 #define PBE_KV_BF16 0
@@ -331,8 +334,7 @@ int pbe_paged_decode(const pbe_arena_view* kv, int32_t kv_dtype, const float* sc
  * capture, tight serving loops, harnesses that forbid hipMalloc). The split-K
  * partials live in a static device array of PBE_DECODE_SCRATCH_BYTES per GPU
  * (held until the process ends) instead of a caller workspace; nothing is
- * allocated and every partial is rewritten by each call, so no clearing is
- * needed. splits = 0 takes pbe_paged_decode_splits' count, lowered until the
+ * allocated and nothing in it needs clearing. splits = 0 takes pbe_paged_decode_splits' count, lowered until the
  * partials fit the array; an explicit split count whose partials need more
  * (pbe_paged_decode_workspace_bytes) is rejected with PBE_ERR_INVALID, as is a
  * batch too large for the array even at one split. All calls on

@@ -48,18 +48,11 @@ extern "C" {
 int32_t pbe_paged_decode_splits(int32_t batch, int32_t kv_heads, int32_t max_blocks_per_seq,
                                 int32_t kv_dtype) {
   if (batch <= 0 || kv_heads <= 0 || max_blocks_per_seq <= 0) return 1;
-  // One wave per SIMD (4 per CU) of the current GPU, rounded down so no
-  // partial extra round of waves trails the launch; FP8 pages take two per
-  // SIMD when every split still holds at least 8 blocks; at least 4 blocks
-  // (64 tokens) per split. Measured on MI355X (256 CUs), FP8, both launches:
-  // 5040-token sequences, batch 64: 16 splits 39.1 us against 40.9 us at 8;
-  // batch 32: 32 splits 26.7 us against 30.2 us at 16; batch 128: 8 splits
-  // 65.9 us against 84.1 us at 4 and 72.9 us at 16; batch 16: 32 splits
-  // 20.9 us, 20.7 us at 64. 2048-token sequences, batch 64: 16 splits 24.6 us
-  // against 27.0 us at 8 and 28.1 us at 32. One 160,000-token sequence (10,000
-  // blocks): 1024 splits 29.5 us against 31.6 us at 512. BF16 batch 64: 54.6
-  // us stage 1 at 8 splits against 56.5 us at 16. One 32768-token sequence:
-  // 512 splits (4 blocks each) 12.0 + 5.9 us against 13.5 + 4.7 at 256.
+  // What the workspace is sized for: the launch cuts the batch into at most
+  // batch * splits slots, and itself takes fewer where that is faster
+  // (decode_kernels.hip). One wave per SIMD (4 per CU) of the current GPU,
+  // rounded down; FP8 pages take two per SIMD when every split still holds at
+  // least 8 blocks; at least 4 blocks (64 tokens) per split.
   const int64_t simds = 4ll * decode_cus();
   const int64_t units = (int64_t)batch * kv_heads;
   int64_t splits = std::max<int64_t>(1, simds / units);
@@ -274,10 +267,6 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
       p.wscales = fp8 ? append_scales : nullptr;
     }
   }
-  const uint64_t rows = (uint64_t)batch * q_heads * splits;
-  p.part_acc = static_cast<float*>(workspace);
-  p.part_m = p.part_acc + rows * shape->head_dim;
-  p.part_l = p.part_m + rows;
   p.batch = batch;
   p.q_heads = q_heads;
   p.kv_heads = shape->kv_heads;
@@ -285,7 +274,7 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   p.layers = shape->layers;
   p.layer = layer;
   p.max_blocks = max_blocks_per_seq;
-  p.splits = splits;
+  pbe::plan_decode_slots(&p, fp8, splits, workspace, need);
   p.half = half;
   p.scale = (1.f / std::sqrt((float)shape->head_dim)) * 1.4426950408889634f;  // as launch_fp8_stage1
   // Largest id whose rows fit: page-major, the whole page (all 2*layers

@@ -8,7 +8,7 @@ namespace pbe {
 
 constexpr int kDecodeMaxSegments = 16;
 constexpr int kDecodeMaxKvMul = 8;    // query heads per KV head held in registers
-constexpr int kDecodeMaxSplits = 1024;  // split weights of one row held in LDS by the combine
+constexpr int kDecodeMaxSplits = 1024;  // slots of one sequence
 
 struct DecodeView {
   const char* base[kDecodeMaxSegments];
@@ -31,10 +31,15 @@ struct DecodeParams {
   uint16_t* out;           // bf16 [batch][q_heads][head_dim]
   const int32_t* tables;   // [batch][max_blocks] page-major block ids
   const int32_t* seq_lens; // [batch]
-  float* part_acc;         // [batch][q_heads][splits][head_dim]
-  float* part_m;           // [batch][q_heads][splits]
-  float* part_l;           // [batch][q_heads][splits]
-  int32_t batch, q_heads, kv_heads, head_dim, layers, layer, max_blocks, splits;
+  // Partial results of the slots (see decode_kernels.hip) of sequences that
+  // take more than one, and their arrival tickets.
+  float* part_acc;         // [slots][q_heads][head_dim]
+  float* part_ml;          // [slots][q_heads][2]: maximum, sum
+  uint64_t* tickets;       // [slots][kv_heads >> hshift]
+  uint64_t tag;            // of this launch (decode_tag())
+  int32_t slots;           // >= batch; == batch: one slot per sequence, no partials
+  int32_t hshift;          // log2 of the KV heads read by one workgroup
+  int32_t batch, q_heads, kv_heads, head_dim, layers, layer, max_blocks;
   uint64_t half;           // bytes of one K or V plane of one block
   int64_t v_delta;         // V rows of a block relative to its K rows (bytes): half page-major
   int64_t vscale_delta;    // V scales relative to K scales (floats): one plane page-major
@@ -53,8 +58,12 @@ struct DecodeParams {
   float* wscales;
 };
 
-// Bytes of the split-K workspace (partial outputs, maxima and sums).
+// Bytes of a workspace that holds the partials of `splits` slots per sequence.
 uint64_t decode_workspace_bytes(int32_t batch, int32_t q_heads, int32_t head_dim, int32_t splits);
+
+// Lays the slots out in `bytes` bytes at `workspace` (at least
+// decode_workspace_bytes(.., splits) of them) and sets p.part_acc .. p.hshift.
+void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes);
 
 hipError_t launch_paged_decode(const DecodeParams& p, bool fp8, hipStream_t stream);
 

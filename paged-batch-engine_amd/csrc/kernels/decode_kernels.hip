@@ -6,15 +6,18 @@
 // score = (q . k) * (log2(e)/sqrt(D) * k_scale), online softmax in base 2,
 // acc += v * (p * v_scale), output = acc / sum as BF16 (round to nearest even).
 //
-// gfx950 mapping. One wave owns one (sequence, KV head, split) and walks its
-// blocks of 16 tokens; the KV heads of one (sequence, split) are neighbouring
-// waves of a workgroup, so a block's rows are read together:
+// gfx950 mapping. The batch's blocks of 16 tokens are cut into slots of about
+// equal length, however long each sequence is (find_slot). A workgroup of 8
+// waves takes one slot for one or two KV heads; the waves of a KV head take
+// the slot's blocks in turn, and the KV heads of a block are read by
+// neighbouring waves:
 //  - loads: a key load instruction covers 64 contiguous bytes of each of the
 //    16 rows (the MFMA wants one row per lane). A value load instruction
 //    covers whole rows, i.e. full 128-byte lines, since the value tile is
 //    rearranged in LDS anyway; requesting half lines instead costs 10% of
-//    the BF16 step. 2 to 8 register sets rotate so that the next blocks are
-//    in flight while one is computed.
+//    the BF16 step. Two register sets take turns: the next block is in flight
+//    while one is computed. The queries lie in LDS, which keeps the wave at
+//    128 registers or fewer, so that two workgroups share a compute unit.
 //  - scores, transposed: one v_mfma_f32_16x16x32_bf16 per 32 head dims,
 //    A = the block's 16 keys (rows), B = the query heads sharing the KV head
 //    (columns, padded to 16). FP8 keys become BF16 exactly (an E4M3 value has
@@ -27,7 +30,18 @@
 //    with ds_read_b64_tr_b8 / _b16, four tokens of one head dim per lane, as
 //    the A operand of O^T += V^T P^T (P^T as held, split into a BF16 high and
 //    low part, K = 32).
-// A second kernel combines the splits.
+//  - results: the waves of a KV head are combined through LDS, and the slots
+//    of a sequence by the workgroup that finishes last (tickets below), in
+//    slot order, so the result does not depend on which one that is.
+//
+// What bounds it: large batches the HBM rate (64 sequences of 5,040 tokens,
+// 2 KV heads x 128: FP8 36.8 us, 4.6 TB/s over the call; the loop alone reads
+// at 6.3), small ones the chain of dependent reads (arguments, lengths, block
+// table, rows, partials, ticket, partials: 1 x 5,040 tokens, 2 x 64 BF16,
+// 10.6 us). Two launches with an equal split count for every sequence took,
+// in the same order, 37.8 and 11.0; 64 sequences of mixed lengths up to 7,040
+// BF16 62.1 (now 40.5); a layer of 8 mixed up to 16,384, 4 x 128 FP8, 30.2
+// (21.3).
 //
 // Append variant (kAppend): the step's new token of every sequence, at its
 // last position, is written into its page slot by the one wave that reads
@@ -36,6 +50,10 @@
 // from its registers rather than from memory, so no ordering between the
 // store and any load is needed, and the result equals writing the row first
 // and reading the pages afterwards, byte for byte.
+#include <algorithm>
+#include <atomic>
+#include <random>
+
 #include "decode_kernels.h"
 #include "fp8_device.h"
 
@@ -47,39 +65,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
+template <typename T>
+using gptr = __attribute__((address_space(1))) T*;  // global memory
+
 constexpr int kBlockTokens = 16;
+constexpr int kStream = 0x02;  // buffer load policy: non-temporal
 
 template <int kCtrl>
 __device__ __forceinline__ float dpp(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xf, 0xf, false));
-}
-
-// Reductions over the 16 lanes of a DPP row: quad_perm [1,0,3,2],
-// quad_perm [2,3,0,1], row_half_mirror, row_mirror.
-__device__ __forceinline__ float row_max16(float x) {
-  x = fmaxf(x, dpp<0xb1>(x));
-  x = fmaxf(x, dpp<0x4e>(x));
-  x = fmaxf(x, dpp<0x141>(x));
-  return fmaxf(x, dpp<0x140>(x));
-}
-
-__device__ __forceinline__ float row_sum16(float x) {
-  x += dpp<0xb1>(x);
-  x += dpp<0x4e>(x);
-  x += dpp<0x141>(x);
-  return x + dpp<0x140>(x);
-}
-
-__device__ __forceinline__ float wave_max(float x) {
-  x = row_max16(x);
-  x = fmaxf(x, __shfl_xor(x, 16));
-  return fmaxf(x, __shfl_xor(x, 32));
-}
-
-__device__ __forceinline__ float wave_sum(float x) {
-  x = row_sum16(x);
-  x += __shfl_xor(x, 16);
-  return x + __shfl_xor(x, 32);
 }
 
 // Max / sum over the four lanes j, j+16, j+32, j+48 with the gfx950 row
@@ -141,61 +135,308 @@ struct BlockRegs {
   float scale;
 };
 
-constexpr int kDecodeWaves = 4;
+constexpr int kWavesLog = 3, kWaves = 1 << kWavesLog, kThreads = 64 * kWaves;  // of a workgroup
+// Slots of one sequence that one workgroup combines in one go; more of them
+// are combined in two levels, groups of about the square root first.
+constexpr int kCombineDirect = 64;
+constexpr int kWorkgroups = 256;  // one per compute unit
+// A sequence of at most kWhole blocks stays whole; a longer one is cut into
+// slots of at least min_chunk blocks (a row: one token of one KV head). us:
+// 64 mixed up to 19 blocks, BF16 x 128, 9.8 whole against 11.0; 10 x 47 blocks
+// of 256-byte rows 11.8 in slots of 8 against 13.1 of 16, 1 x 315 of 128-byte
+// rows 12.0 against 11.3.
+constexpr int kWhole = 24;
+constexpr int min_chunk(int row_bytes) { return row_bytes >= 256 ? 8 : 16; }
 
-// kSets register sets per wave: kSets-1 blocks in flight while one is
-// computed (chosen at launch, see sets_for).
-template <int D, bool kFp8, int KVM, bool kAppend, int kSets>
-__global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
-    const DecodeParams p, const int32_t* __restrict__ tables) {
+// ---- which blocks a workgroup reads ---------------------------------------
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int scan_step(int x) {
+  return x + __builtin_amdgcn_update_dpp(0, x, kCtrl, kRows, 0xf, false);
+}
+// Inclusive prefix sum over the wave's lanes.
+__device__ __forceinline__ int wave_scan(int x) {
+  x = scan_step<0x111, 0xf>(x);  // row_shr 1, 2, 4, 8: within rows of 16
+  x = scan_step<0x112, 0xf>(x);
+  x = scan_step<0x114, 0xf>(x);
+  x = scan_step<0x118, 0xf>(x);
+  x = scan_step<0x142, 0xa>(x);     // row_bcast 15 into rows 1 and 3
+  return scan_step<0x143, 0xc>(x);  // row_bcast 31 into rows 2 and 3
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+template <int kCtrl>
+__device__ __forceinline__ int max_step(int x) {
+  return max(x, __builtin_amdgcn_update_dpp(x, x, kCtrl, 0xf, 0xf, false));
+}
+__device__ __forceinline__ int wave_max_int(int x) {
+  x = max_step<0xb1>(x);
+  x = max_step<0x4e>(x);
+  x = max_step<0x141>(x);
+  x = max_step<0x140>(x);
+  return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+             max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
+
+// Blocks of a length; a bad one (negative, or beyond the table) has none.
+__device__ __forceinline__ int blocks_of(int seq, int max_blocks) {
+  const int n = seq > 0 ? (int)(((uint32_t)seq + kBlockTokens - 1) / kBlockTokens) : 0;
+  return n <= max_blocks ? n : 0;
+}
+// Slots of a sequence of n blocks at c blocks per slot.
+__device__ __forceinline__ int slots_of(int n, uint32_t c) {
+  return n <= kWhole ? 1 : (int)(((uint32_t)n + c - 1) / c);
+}
+
+// One slot: a chunk of one sequence's blocks. The chunk length c is the same
+// for the whole batch, so a batch of mixed lengths keeps every workgroup
+// equally busy: a sequence of n blocks takes max(1, ceil(n / c)) slots, c
+// being about the shortest (at least min_chunk) whose slots fit the slots of
+// the launch. The lengths are device memory, so each workgroup works this out
+// for itself: its waves try one c each, then find their slot with a prefix
+// scan over the batch. (A binary search in every wave took 3.6 us of a batch
+// of 160, 10 us with two workgroups per compute unit; this takes 1.6 and 3.)
+//
+// How many slots (W = kWorkgroups / workgroups per slot = one per compute
+// unit; us on MI355X, 2 KV heads x 128 unless said otherwise):
+//  - batch < W: W slots. Twice as many (two workgroups per compute unit) read
+//    64 x 5,040 tokens in 65.0 against 57.7 (BF16), 39.2 against 37.8 (FP8):
+//    the second set's slots start and end at the same time as the first's.
+//    But where rows are 128 bytes or less (one workgroup's loads in flight
+//    then do not saturate its compute unit) and W slots would leave a quarter
+//    of the chip idle (160 equal sequences: 160 slots), 2W: FP8 160 x 2,000
+//    tokens 41.4 against 45.7. BF16 rows of 256 bytes gain nothing: 160
+//    mixed up to 1,000 tokens 29.5 against 26.1.
+//  - batch >= W: a sequence is split only where it is longer than 5/4 of the
+//    mean. FP8 256 x 1,000 equal lengths 30.5 against 36.6 with two slots
+//    each, BF16 256 mixed up to 1,000 42.4 against 51.1 with W/2 more slots
+//    than sequences.
+struct Slot {
+  int b = -1;  // sequence; -1: no work for this workgroup
+  int seq = 0;
+  int k = 1, s = 0;  // the sequence's slots, and which of them this is
+  int per = 1;       // blocks per slot
+};
+
+// `z`: this workgroup's slot; `slots` of the launch; `fit`: LDS.
+template <int kMin>
+__device__ __forceinline__ Slot find_slot(uint32_t (*fit)[kWaves], const int32_t* __restrict__ lens, int batch,
+                                          int max_blocks, int slots, int one_round, int z, int w, int lane) {
+  Slot r;
+  if (slots == batch) {
+    r.b = z;
+    r.seq = lens[z];
+    r.per = max(1, blocks_of(r.seq, max_blocks));
+    return r;
+  }
+  // A lane's sequences are lane, lane + 64, ...; the first few stay in registers.
+  constexpr int kKept = 4;
+  int seqs[kKept], kept[kKept], sum = 0, most = 0;
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) seqs[i] = lane + 64 * i < batch ? lens[lane + 64 * i] : 0;
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) {
+    kept[i] = blocks_of(seqs[i], max_blocks);
+    sum += kept[i];
+    most = max(most, kept[i]);
+  }
+  for (int i = lane + 64 * kKept; i < batch; i += 64) {
+    const int n = blocks_of(lens[i], max_blocks);
+    sum += n;
+    most = max(most, n);
+  }
+  const uint32_t total = (uint32_t)wave_total(sum), longest = (uint32_t)wave_max_int(most);
+  auto count = [&](uint32_t c) {
+    int x = 0;
+#pragma unroll
+    for (int i = 0; i < kKept; ++i)
+      if (64 * i < batch) x += lane + 64 * i < batch ? slots_of(kept[i], c) : 0;
+    for (int i = lane + 64 * kKept; i < batch; i += 64) x += slots_of(blocks_of(lens[i], max_blocks), c);
+    return wave_total(x);
+  };
+  const bool many = batch >= one_round;
+  const uint32_t mean = many ? total / (uint32_t)batch : 0u;
+  auto chunk = [&](uint32_t T, int round) {
+    // sum of ceil(n/c) <= total/c + batch, so c >= total/(T - batch) fits
+    const uint32_t extra = T - (uint32_t)batch;
+    if (!many && (uint64_t)total <= (uint64_t)extra * kMin && longest <= (uint32_t)(kDecodeMaxSplits * kMin)) return (uint32_t)kMin;
+    const uint32_t lo = max(max((total + T - 1) / T, (longest + kDecodeMaxSplits - 1) / kDecodeMaxSplits),
+                            max(mean + mean / 4, (uint32_t)kMin));
+    const uint32_t hi = max(lo, min(max(1u, longest), (total + extra - 1) / extra));
+    if (lo == hi) return lo;
+    const uint32_t c = lo + (uint32_t)((uint64_t)w * (hi - lo) / kWaves);
+    const bool fits = count(c) <= (int)T;
+    if (lane == 0) fit[round][w] = fits ? c : hi;
+    __syncthreads();
+    uint32_t best = hi;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) best = min(best, fit[round][i]);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)best);
+  };
+  uint32_t c = 0;
+  for (int round = 0; round < 2; ++round) {
+    c = chunk((uint32_t)(many || round ? slots : min(slots, one_round)), round);
+    const bool idle = !many && slots > one_round && c > (uint32_t)kMin &&
+                      (uint64_t)total * 4 < (uint64_t)c * (uint32_t)one_round * 3;
+    if (!idle) break;
+  }
+  // the sequence whose slots hold z; the other workgroups have nothing to do
+  int before = 0;
+  for (int i = 0; i < batch; i += 64) {
+    int seq = seqs[0];
+#pragma unroll
+    for (int e = 1; e < kKept; ++e) seq = i == 64 * e ? seqs[e] : seq;
+    if (i >= 64 * kKept) seq = i + lane < batch ? lens[i + lane] : 0;
+    const int n = blocks_of(seq, max_blocks);
+    const int k = i + lane < batch ? slots_of(n, c) : 0;
+    const int upto = wave_scan(k) + before;
+    const uint64_t past = __ballot(upto > z);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      r.b = i + at;
+      r.seq = __builtin_amdgcn_readlane(seq, at);
+      r.k = __builtin_amdgcn_readlane(k, at);
+      r.s = z - (__builtin_amdgcn_readlane(upto, at) - r.k);
+      const int nb = __builtin_amdgcn_readlane(n, at);
+      r.per = max(1, (nb + r.k - 1) / r.k);        // even slots ...
+      r.k = slots_of(nb, (uint32_t)r.per);         // ... which may need fewer of them
+      if (r.s >= r.k) r.b = -1;
+      return r;
+    }
+    before = __builtin_amdgcn_readlane(upto, 63);
+  }
+  return r;
+}
+
+// ---- partial results between workgroups -----------------------------------
+// A slot's partial (fp32 output, maximum and sum) is written and read at
+// agent scope (relaxed atomics: written through, read past the XCD's own L2),
+// so no L2 write-back or invalidate is needed: the writer waits for its
+// stores to complete, then takes a ticket; whoever takes the last one reads.
+constexpr int kAgent = 0x10;  // buffer access policy: agent scope
+
+// Arrival tickets. A word holds tag << kTicketBits | arrivals of launch `tag`;
+// anything else in it (a workspace may hold anything) counts as none. The last
+// arrival leaves 0, so a replayed launch, which has the same tag, starts anew.
+constexpr int kTicketBits = 11;
+static_assert(kDecodeMaxSplits < (1 << kTicketBits), "arrivals fit the ticket");
+// Makes a word that is 0 ready for arrivals; nothing waits for it.
+__device__ __forceinline__ void open_ticket(gptr<uint64_t> word, uint64_t tag) {
+  uint64_t none = 0;
+  (void)__hip_atomic_compare_exchange_strong(word, &none, tag << kTicketBits, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+}
+// Whether this is the last of `members` arrivals: one round trip where the
+// word was opened; a word that held something else is claimed by exchange.
+__device__ __forceinline__ bool last_arrival(gptr<uint64_t> word, uint64_t tag, uint32_t members) {
+  uint64_t now = __hip_atomic_fetch_add(word, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+  if ((now >> kTicketBits) != tag) {
+    uint64_t seen = now;
+    do {
+      now = (seen >> kTicketBits) == tag ? seen + 1 : (tag << kTicketBits) | 1u;
+    } while (!__hip_atomic_compare_exchange_strong(word, &seen, now, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT));
+  }
+  if ((now & ((1u << kTicketBits) - 1)) != members) return false;
+  __hip_atomic_store(word, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// One head's running combination of partials: maximum, sum and output, the
+// latter two weighted by 2^(m_i - m) (paged_mha_fast_kernel.cu:730-799). A NaN
+// sum stays NaN; a partial of weight 0 is left out whatever its output holds.
+struct Combined {
+  float m = -INFINITY, l = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  __device__ __forceinline__ void raise(float top) {  // to a maximum top >= m
+    const float scale = l > 0.f ? __builtin_amdgcn_exp2f(m - top) : 0.f;
+    l = l != l ? l : l * scale;
+    acc = scale > 0.f ? acc * scale : f32x4{0.f, 0.f, 0.f, 0.f};
+    m = top;
+  }
+  __device__ __forceinline__ void weigh(float m_i, float l_i, const f32x4& acc_i) {  // m_i <= m
+    const float wt = l_i > 0.f ? __builtin_amdgcn_exp2f(m_i - m) : 0.f;
+    l += l_i != l_i ? l_i : l_i * wt;
+    if (wt > 0.f) acc += acc_i * wt;
+  }
+};
+
+// ---- the kernel -------------------------------------------------------------
+template <int D, bool kFp8, int KVM, bool kAppend>
+__global__ __launch_bounds__(kThreads, 4) void paged_decode_kernel(
+    const int32_t* __restrict__ lens, const int32_t* __restrict__ tables, const int batch, const int max_blocks, const int slots,
+    const int hshift, const uint32_t groups_d, const uint32_t groups_mul, const uint32_t groups_shift,
+    const DecodeParams p) {
   using G = Geo<D, kFp8>;
   constexpr int E = G::E;
   constexpr int NK = D / 32;  // score MFMAs per block
   constexpr int NT = D / 16;  // value MFMAs (16 head dims each) per block
-  constexpr int W = G::WORDS, SETS = kSets, PITCH = G::PITCH;
-  __shared__ __attribute__((aligned(16))) unsigned char lds_v[kDecodeWaves][kBlockTokens * PITCH];
+  constexpr int W = G::WORDS, PITCH = G::PITCH;
+  constexpr int OUT_PITCH = D + 4;  // floats; the pad spreads the heads over the banks
+  constexpr int kTile = kBlockTokens * PITCH, kOut = KVM * OUT_PITCH * 4;
+  constexpr int kTeams = 64 * 24;  // what a wave's threads exchange when they share slots
+  constexpr int kWaveLds = kTile > kOut ? (kTile > kTeams ? kTile : kTeams) : (kOut > kTeams ? kOut : kTeams);
+  // value tiles while blocks are read, then the waves' outputs
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves][kWaveLds];
+  __shared__ float lds_m[kWaves][16], lds_l[kWaves][16];
+  __shared__ int lds_last[2];
+  __shared__ uint32_t fit[2][kWaves];
+  __shared__ __attribute__((aligned(16))) unsigned char lds_new[kAppend ? kWaves : 1][kAppend ? 2 * D * E : 16];
+  __shared__ bf16x8 lds_q[kWaves][NK][64];
 
+  // The arguments that follow the preloaded ones, read in one go: left to
+  // itself the compiler reads each where it is used, one scalar round trip
+  // after another.
+  gptr<const char> kv0 = (gptr<const char>)p.kv.base[0];
+  gptr<const float> scales = (gptr<const float>)p.scales;
+  gptr<const uint16_t> q_rows = (gptr<const uint16_t>)p.q;
+  gptr<uint16_t> out = (gptr<uint16_t>)p.out;
+  gptr<float> part_acc = (gptr<float>)p.part_acc, part_ml = (gptr<float>)p.part_ml;
+  gptr<uint64_t> tickets = (gptr<uint64_t>)p.tickets;
+  uint64_t tag = p.tag, half = p.half;
+  int64_t v_delta = p.v_delta, vscale_delta = p.vscale_delta;
+  int q_heads = p.q_heads, layer = p.layer, id_max = p.id_max;
+  float score_scale = p.scale;
+  FastDiv by_stride = p.by_stride, by_seg_pages = p.by_seg_pages;
+  asm volatile("" : "+s"(kv0), "+s"(q_rows), "+s"(out), "+s"(part_acc), "+s"(part_ml), "+s"(tickets), "+s"(tag), "+s"(half),
+               "+s"(v_delta), "+s"(q_heads), "+s"(layer), "+s"(id_max), "+s"(score_scale), "+s"(by_stride.d),
+               "+s"(by_stride.mul), "+s"(by_stride.shift), "+s"(by_seg_pages.d), "+s"(by_seg_pages.mul), "+s"(by_seg_pages.shift));
+  if constexpr (kFp8) asm volatile("" : "+s"(scales), "+s"(vscale_delta));
+  gptr<const uint16_t> new_k = nullptr, new_v = nullptr;
+  gptr<char> kv0_w = nullptr;
+  gptr<float> wscales = nullptr;
+  if constexpr (kAppend) {
+    new_k = (gptr<const uint16_t>)p.new_k, new_v = (gptr<const uint16_t>)p.new_v;
+    kv0_w = (gptr<char>)p.wbase[0], wscales = (gptr<float>)p.wscales;
+    asm volatile("" : "+s"(new_k), "+s"(new_v), "+s"(kv0_w), "+s"(wscales));
+  }
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t unit = (int64_t)blockIdx.x * kDecodeWaves + w;
-  if (unit >= (int64_t)p.batch * p.kv_heads * p.splits) return;
-  const int kvh = (int)(unit % p.kv_heads);
-  const int split = (int)((unit / p.kv_heads) % p.splits);
-  const int b = (int)(unit / p.kv_heads / p.splits);
+  const int head_groups = (int)groups_d, kv_heads = head_groups << hshift;
+  const int z = (int)fast_div(blockIdx.x, FastDiv{groups_d, groups_mul, groups_shift});
+  const int hg = (int)blockIdx.x - z * head_groups;
+  const Slot slot = find_slot<min_chunk(D * E)>(fit, lens, batch, max_blocks, slots, max(1, kWorkgroups / head_groups), z, w, lane);
+  if (slot.b < 0) return;
+  const int b = slot.b, seq = slot.seq;
+  // Of the workgroup's waves, every (1 << hshift)th reads the same KV head:
+  // the KV heads of a token row are read together, by neighbouring waves.
+  const int hw = 1 << hshift, sub_shift = kWavesLog - hshift, subs = 1 << sub_shift;
+  const int hloc = w & (hw - 1), sub = w >> hshift;
+  const int kvh = (hg << hshift) + hloc;
   const int g = lane >> 4, j = lane & 15;
-  const int seq = p.seq_lens[b];
-  const int nblk = seq > 0 ? (seq + kBlockTokens - 1) / kBlockTokens : 0;
-  bool bad = seq < 0 || nblk > p.max_blocks;
-  // Each sequence's blocks are cut into `splits` equal ranges
-  // (paged_mha_fast_kernel.cu:596-601).
-  const int per_split = (nblk + p.splits - 1) / p.splits;
-  const int blk0 = split * per_split;
-  int blk1 = bad ? blk0 : min(blk0 + per_split, nblk);
+  const int nblk = seq > 0 ? (int)(((uint32_t)seq + kBlockTokens - 1) / kBlockTokens) : 0;
+  bool bad = seq < 0 || nblk > max_blocks;
+  // The slot's blocks, dealt to the waves of a KV head in turn.
+  const int chunk0 = slot.s * slot.per;
+  const int blk0 = chunk0 + sub;
+  int blk1 = bad ? chunk0 : min(chunk0 + slot.per, nblk);
 
-  // Query rows as the B operand of the scores: lane (g, j) holds head j's
-  // dims matching the key bytes MFMA kk consumes (rows past the group's
-  // heads are zero).
-  bf16x8 qa[NK];
-  {
-    const bool has = j < KVM;
-    const uint16_t* qrow =
-        p.q + ((int64_t)b * p.q_heads + (int64_t)kvh * KVM + (has ? j : 0)) * D;
-#pragma unroll
-    for (int kk = 0; kk < NK; ++kk) {
-      // the head dims of the key bytes this MFMA consumes (see key_off)
-      const int cb = kk * 8 * E;
-      const int dim0 = (64 / E) * (cb / 16) + (16 / E) * g + (cb % 16) / E;
-      const u32x4 v = has ? *reinterpret_cast<const u32x4*>(qrow + dim0) : u32x4{0u, 0u, 0u, 0u};
-      qa[kk] = __builtin_bit_cast(bf16x8, v);
-    }
-  }
-
-  const uint64_t H = (uint64_t)p.kv_heads;
+  const uint64_t H = (uint64_t)kv_heads;
   const uint32_t token_stride = (uint32_t)(H * D * E);
-  const uint64_t stride = p.by_stride.d;
-  // Block ids are uniform: read through the read-only table with scalar loads.
-  const int32_t* table = tables + (int64_t)b * p.max_blocks;
-  const uint64_t head_off = 2ull * p.layer * p.half + (uint64_t)kvh * D * E;
+  const uint64_t stride = by_stride.d;
+  // The wave's next 64 block ids, one per lane (a vector load every 64 blocks
+  // instead of a scalar round trip before each).
+  gptr<const int32_t> table = (gptr<const int32_t>)tables + (int64_t)b * max_blocks;
+  int32_t window = table[min(blk0 + (lane << sub_shift), max_blocks - 1)];
+  const uint64_t head_off = 2ull * layer * half + (uint64_t)kvh * D * E;
   // Key load v of lane (g, j) reads bytes 64v + 16g.. of key row j: 64
   // contiguous bytes of every row per instruction. The key's head dims are
   // consumed in that order; the queries are read in the same order.
@@ -208,52 +449,71 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
   const uint32_t val_off = (uint32_t)vrow0 * token_stride + (uint32_t)vcol;
   // lane (g, j): scale of token 4g + j%4 from the key (j%8 < 4) or value plane
   const int64_t scale_off =
-      (int64_t)((2u * p.layer * kBlockTokens + 4u * g + (j & 3)) * H + kvh) + ((j >> 2) & 1 ? p.vscale_delta : 0);
+      (int64_t)((2u * layer * kBlockTokens + 4u * g + (j & 3)) * H + kvh) + ((j >> 2) & 1 ? vscale_delta : 0);
+  const uint32_t row_span = (uint32_t)(half - (uint64_t)kvh * D * E);  // this head's rows, to the plane's end
   // Loads block `blk` into `r`. Every call issues the same loads (an
-  // unconditional count keeps the compiler's in-flight accounting exact): a
-  // block past the split's end, or whose id is not a page id inside the arena
-  // and scale pool, reads page 0 instead and reports false when it was wanted.
+  // unconditional count keeps the compiler's in-flight accounting exact), but
+  // a block past the split's end, or whose id is not a page id inside the
+  // arena and scale pool, is an empty buffer: its row loads return zeros and
+  // read no memory (the scale load reads a row of block 0). Reports false
+  // when such a bad block was wanted.
   auto load = [&](int blk, BlockRegs<W, kFp8>& r) -> bool {
     const bool want = blk < blk1;
-    int32_t id = want ? table[blk] : 0;
-    uint32_t page = fast_div((uint32_t)max(id, 0), p.by_stride);
-    const bool ok = id >= 0 && id <= p.id_max && page * p.by_stride.d == (uint32_t)id;
+    const int at = (blk - blk0) >> sub_shift;
+    if (at && (at & 63) == 0) window = table[min(blk + (lane << sub_shift), max_blocks - 1)];
+    int32_t id = want ? __builtin_amdgcn_readlane(window, at & 63) : 0;
+    uint32_t page = fast_div((uint32_t)max(id, 0), by_stride);
+    const bool ok = id >= 0 && id <= id_max && page * by_stride.d == (uint32_t)id;
     if (!ok) id = 0, page = 0;
-    const uint32_t seg = fast_div(page, p.by_seg_pages);
-    const char* kplane =
-        p.kv.base[seg] + (uint64_t)(page - seg * p.by_seg_pages.d) * stride * p.half + head_off;
+    const uint32_t seg = fast_div(page, by_seg_pages);
+    gptr<const char> kplane =
+        (seg ? (gptr<const char>)p.kv.base[seg] : kv0) + (uint64_t)(page - seg * by_seg_pages.d) * stride * half + head_off;
+    const uint32_t span = want && ok ? row_span : 0u;
+    const __amdgpu_buffer_rsrc_t rk =
+        __builtin_amdgcn_make_buffer_rsrc((void*)kplane, (short)0, span, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(kplane + v_delta), (short)0, span, 0x00020000);
+    uint32_t val_step = RPI * token_stride;
+    asm volatile("" : "+s"(val_step));  // added per block: the offsets would take W/4 registers
 #pragma unroll
     for (int v = 0; v < W / 4; ++v) {
-      const u32x4 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kplane + key_off + 64 * v));
-      const u32x4 y = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4*>(kplane + p.v_delta + val_off + (uint64_t)v * RPI * token_stride));
+      const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rk, key_off + 64 * v, 0, kStream);
+      const u32x4 y = __builtin_amdgcn_raw_buffer_load_b128(rv, val_off + (uint32_t)v * val_step, 0, kStream);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         r.k[4 * v + e] = x[e];
         r.v[4 * v + e] = y[e];
       }
     }
-    if constexpr (kFp8) {  // key scales carry the score scale: p.scale * k_scale
+    if constexpr (kFp8) {  // key scales carry the score scale: score_scale * k_scale
       // Non-temporal like the page rows: plain loads cost 8% of the FP8 step.
-      const float sc = __builtin_nontemporal_load(p.scales + (uint64_t)id * kBlockTokens * H + scale_off);
-      r.scale = (j & 4) ? sc : p.scale * sc;
+      const float sc = __builtin_nontemporal_load(scales + (uint64_t)id * kBlockTokens * H + scale_off);
+      r.scale = (j & 4) ? sc : score_scale * sc;
     }
     return ok || !want;
   };
 
+  // Slots of one sequence are combined in groups, and the groups after them.
+  int group = slot.k, groups = 1, gi = 0;
+  if (slot.k > kCombineDirect) {
+    group = 8;
+    while (group * group < slot.k) group += 4;
+    groups = (slot.k + group - 1) / group;
+    gi = slot.s / group;
+  }
+  const int z0 = z - slot.s;  // the sequence's first slot
+  const int zg = z0 + gi * group, in_group = min(group, slot.k - gi * group);
   float m = -INFINITY, l = 0.f;  // of head j
   f32x4 acc[NT];                 // O^T: lane (g, j) = head j, dims 16nt + 4g + 0..3
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Append: the new token's row of this KV head as lane (g, j) holds key row
-  // j (nk), as the value writer lanes computed it (nv), its scales, and the
-  // block it lands in (-1: nothing to write here).
-  uint32_t nk[kAppend ? W : 1], nv[kAppend ? 4 : 1];
+  // Append: the new token's row of this KV head lies in lds_new (keys, then
+  // values); its scales, and the block it lands in (-1: nothing to write here).
   float nks = 0.f, nvs = 0.f;
   int patch_blk = -1, slot_row = 0;
 
-  unsigned char* vt_w = &lds_v[w][0];
+  unsigned char* vt_w = &lds[w][0];
   auto compute = [&](int blk, const BlockRegs<W, kFp8>& r) {
     const int valid = blk == nblk - 1 ? seq - kBlockTokens * (nblk - 1) : kBlockTokens;
     const bool patch = kAppend && blk == patch_blk;
@@ -262,7 +522,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
       unsigned char* dst = vt_w + vrow0 * PITCH + vcol;
 #pragma unroll
       for (int v = 0; v < W / 4; ++v) {
-        const u32x4 x = v * RPI + vrow0 < valid
+        const u32x4 x = vrow0 < valid - v * RPI
                             ? u32x4{r.v[4 * v], r.v[4 * v + 1], r.v[4 * v + 2], r.v[4 * v + 3]}
                             : u32x4{0u, 0u, 0u, 0u};
         *reinterpret_cast<u32x4*>(dst + v * RPI * PITCH) = x;
@@ -271,9 +531,11 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
       // issue order).
       if constexpr (kAppend) {
         if (patch && lane >= 32 && (lane & 31) < RL) {
-          unsigned char* row = vt_w + slot_row * PITCH + (kFp8 ? 8 : 16) * (lane & 31);
-          if constexpr (kFp8) *reinterpret_cast<u32x2*>(row) = u32x2{nv[0], nv[1]};
-          else *reinterpret_cast<u32x4*>(row) = u32x4{nv[0], nv[1], nv[2], nv[3]};
+          const int at = (kFp8 ? 8 : 16) * (lane & 31);
+          unsigned char* row = vt_w + slot_row * PITCH + at;
+          const unsigned char* from = lds_new[w] + D * E + at;
+          if constexpr (kFp8) *reinterpret_cast<u32x2*>(row) = *reinterpret_cast<const u32x2*>(from);
+          else *reinterpret_cast<u32x4*>(row) = *reinterpret_cast<const u32x4*>(from);
         }
       }
     }
@@ -284,10 +546,15 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
     float rscale = kFp8 ? r.scale : 0.f;
     if constexpr (kAppend) {
       if (patch) {
-        const bool mine = j == slot_row;
+        if (j == slot_row) {
 #pragma unroll
-        for (int i = 0; i < W; ++i) kw[i] = mine ? nk[i] : kw[i];
-        if (4 * g + (j & 3) == slot_row) rscale = (j & 4) ? nvs : p.scale * nks;
+          for (int v = 0; v < W / 4; ++v) {
+            const u32x4 x = *reinterpret_cast<const u32x4*>(lds_new[w] + 64 * v + 16 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kw[4 * v + e] = x[e];
+          }
+        }
+        if (4 * g + (j & 3) == slot_row) rscale = (j & 4) ? nvs : score_scale * nks;
       }
     }
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
@@ -301,10 +568,10 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
       } else {
         kb = __builtin_bit_cast(bf16x8, u32x4{kw[4 * kk], kw[4 * kk + 1], kw[4 * kk + 2], kw[4 * kk + 3]});
       }
-      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qa[kk], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, lds_q[w][kk][lane], s, 0, 0, 0);
     }
     wave_sync();
-    float ks[4] = {p.scale, p.scale, p.scale, p.scale}, vs[4] = {1.f, 1.f, 1.f, 1.f};
+    float ks[4] = {score_scale, score_scale, score_scale, score_scale}, vs[4] = {1.f, 1.f, 1.f, 1.f};
     if constexpr (kFp8) {  // broadcast within each 16-lane row
       ks[0] = dpp<0x150>(rscale);
       ks[1] = dpp<0x151>(rscale);
@@ -319,7 +586,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
     float sv[4], tmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      sv[i] = 4 * g + i < valid ? s[i] * ks[i] : -INFINITY;
+      sv[i] = 4 * g < valid - i ? s[i] * ks[i] : -INFINITY;
       tmax = fmaxf(tmax, sv[i]);
     }
     tmax = group_max4(tmax);
@@ -329,7 +596,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
     uint32_t phi[2], plo[2];
 #pragma unroll
     for (int i = 0; i < 4; i += 2) {
-      const bool ok0 = 4 * g + i < valid, ok1 = 4 * g + i + 1 < valid;
+      const bool ok0 = 4 * g < valid - i, ok1 = 4 * g < valid - i - 1;
       const float p0 = ok0 ? __builtin_amdgcn_exp2f(sv[i] - mn) : 0.f;
       const float p1 = ok1 ? __builtin_amdgcn_exp2f(sv[i + 1] - mn) : 0.f;
       psum += p0 + p1;
@@ -383,210 +650,227 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void paged_decode_kernel(
     wave_sync();  // the next block rewrites the tile
   };
 
-  // SETS register sets in rotation: while one block is computed, the next
-  // SETS-1 are in flight.
-  static_assert(SETS >= 2 && SETS <= 8, "2 to 8 register sets");
-  BlockRegs<W, kFp8> r[SETS];
-  auto prime = [&](int blk, BlockRegs<W, kFp8>& rr) {
+  // Append: the wave that reads the sequence's last block takes the new token's
+  // row, lanes 0..RL-1 of the keys and lanes 32..32+RL-1 of the values.
+  const int last = nblk - 1;
+  const bool writer = kAppend && !bad && seq > 0 && last >= chunk0 && last < chunk0 + slot.per && ((last - chunk0) & (subs - 1)) == sub;
+  const bool is_v = lane >= 32, act = (lane & 31) < RL;
+  u32x4 row_in = {0u, 0u, 0u, 0u};
+  if constexpr (kAppend) {
+    if (writer && act)
+      row_in = __builtin_nontemporal_load((gptr<const u32x4>)((is_v ? new_v : new_k) + ((int64_t)b * kv_heads + kvh) * D + 8 * (lane & 31)));
+  }
+  // Query rows as the B operand of the scores: lane (g, j) holds head j's
+  // dims matching the key bytes MFMA kk consumes (rows past the group's
+  // heads are zero).
+  u32x4 q_in[NK];
+  {
+    const bool has = j < KVM;
+    gptr<const uint16_t> qrow = q_rows + ((int64_t)b * q_heads + (int64_t)kvh * KVM + (has ? j : 0)) * D;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      // the head dims of the key bytes this MFMA consumes (see key_off)
+      const int cb = kk * 8 * E;
+      const int dim0 = (64 / E) * (cb / 16) + (16 / E) * g + (cb % 16) / E;
+      q_in[kk] = *(gptr<const u32x4>)(qrow + dim0);
+    }
+  }
+  // Two register sets in turn: while one block is computed, the next is in flight.
+  BlockRegs<W, kFp8> r[2];
+  auto fetch = [&](int blk, BlockRegs<W, kFp8>& rr) {
     if (!load(blk, rr)) bad = true, blk1 = min(blk1, blk);
   };
-  auto step = [&](int blk, BlockRegs<W, kFp8>& rr) {
-    if (blk < blk1) compute(blk, rr);
-    if (!load(blk + SETS, rr)) bad = true, blk1 = min(blk1, blk + SETS);
-  };
+  fetch(blk0, r[0]);
+  fetch(blk0 + subs, r[1]);
 #pragma unroll
-  for (int i = 0; i < SETS; ++i) prime(blk0 + i, r[i]);
+  for (int kk = 0; kk < NK; ++kk) lds_q[w][kk][lane] = __builtin_bit_cast(bf16x8, j < KVM ? q_in[kk] : u32x4{0u, 0u, 0u, 0u});
+  if (slot.k > 1 && threadIdx.x == 0) {
+    open_ticket(tickets + (int64_t)zg * head_groups + hg, tag);
+    if (groups > 1) open_ticket(tickets + (int64_t)(z0 + 1) * head_groups + hg, tag);
+  }
   if constexpr (kAppend) {
-    // The wave whose split holds the sequence's last block writes the new
-    // token there (while its first blocks are in flight). Lanes 0..RL-1 take
-    // the key row, lanes 32..32+RL-1 the value row, 16 input bytes each, as
-    // the page writer does with D/8 lanes per head.
-    const int last = nblk - 1;
-    if (seq > 0 && nblk <= p.max_blocks && last >= blk0 && last < blk0 + per_split) {
-      const int32_t id = table[last];
-      const uint32_t page = fast_div((uint32_t)max(id, 0), p.by_stride);
-      if (id >= 0 && id <= p.id_max && page * p.by_stride.d == (uint32_t)id) {
+    // It writes the row (while its first blocks are in flight) as the page
+    // writer does with D/8 lanes per head.
+    if (writer) {
+      const int at = (last - blk0) >> sub_shift;
+      const int32_t id = at < 64 ? __builtin_amdgcn_readlane(window, at) : table[last];
+      const uint32_t page = fast_div((uint32_t)max(id, 0), by_stride);
+      if (id >= 0 && id <= id_max && page * by_stride.d == (uint32_t)id) {
         const int row = seq - 1 - kBlockTokens * last;
-        const uint32_t seg = fast_div(page, p.by_seg_pages);
-        char* krow = p.wbase[seg] + (uint64_t)(page - seg * p.by_seg_pages.d) * stride * p.half +
-                     head_off + (uint64_t)row * token_stride;
-        const bool is_v = lane >= 32;
+        const uint32_t seg = fast_div(page, by_seg_pages);
+        gptr<char> krow = (seg ? (gptr<char>)p.wbase[seg] : kv0_w) + (uint64_t)(page - seg * by_seg_pages.d) * stride * half +
+                          head_off + (uint64_t)row * token_stride;
         const int li = lane & 31;
-        const bool act = li < RL;
-        const uint16_t* src = (is_v ? p.new_v : p.new_k) + ((int64_t)b * p.kv_heads + kvh) * D + 8 * (act ? li : 0);
-        const u32x4 x = act ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src)) : u32x4{0u, 0u, 0u, 0u};
-        char* dst = krow + (is_v ? p.v_delta : 0);
+        const u32x4 x = row_in;
+        gptr<char> dst = krow + (is_v ? v_delta : 0);
         if constexpr (kFp8) {
           const float mx = group_max<RL>(amax8(x));
           const float inv = mx > 0.f ? 448.f / mx : 0.f;
           const float sc = mx > 0.f ? mx / 448.f : 1.f;
           const u32x2 c = quantise8(x, inv);
-          if (act) *reinterpret_cast<u32x2*>(dst + 8 * li) = c;
+          if (act) *(gptr<u32x2>)(dst + 8 * li) = c;
           if (act && li == 0)
-            p.wscales[(uint64_t)id * kBlockTokens * H +
-                                         (2u * p.layer * kBlockTokens + row) * H + kvh + (is_v ? p.vscale_delta : 0)] = sc;
-          nks = __shfl(sc, 0);
-          nvs = __shfl(sc, 32);
-#pragma unroll
-          for (int i = 0; i < W; ++i) nk[i] = __shfl(c[i & 1], (64 * (i / 4) + 16 * g + 4 * (i % 4)) / 8);
-          nv[0] = c[0];
-          nv[1] = c[1];
+            wscales[(uint64_t)id * kBlockTokens * H +
+                                         (2u * layer * kBlockTokens + row) * H + kvh + (is_v ? vscale_delta : 0)] = sc;
+          nks = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), 0));
+          nvs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), 32));
+          if (act) *reinterpret_cast<u32x2*>(lds_new[w] + (is_v ? D * E : 0) + 8 * li) = c;
         } else {
-          if (act) *reinterpret_cast<u32x4*>(dst + 16 * li) = x;
-#pragma unroll
-          for (int i = 0; i < W; ++i) nk[i] = __shfl(x[i % 4], 4 * (i / 4) + g);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) nv[e] = x[e];
+          if (act) *(gptr<u32x4>)(dst + 16 * li) = x;
+          if (act) *reinterpret_cast<u32x4*>(lds_new[w] + (is_v ? D * E : 0) + 16 * li) = x;
         }
         patch_blk = last;
         slot_row = row;
+        wave_sync();
       }
     }
   }
-  for (int base = blk0; base < blk1; base += SETS) {
-#pragma unroll
-    for (int i = 0; i < SETS; ++i) step(base + i, r[i]);
+  for (int blk = blk0; blk < blk1; blk += 2 * subs) {
+    compute(blk, r[0]);
+    fetch(blk + 2 * subs, r[0]);
+    if (blk + subs < blk1) compute(blk + subs, r[1]);
+    fetch(blk + 3 * subs, r[1]);
   }
 
-  // ---- this split's partials (lane (g, j): head j, dims 16nt + 4g + i)
-  const int64_t row0 = (int64_t)b * p.q_heads + (int64_t)kvh * KVM;
-  const float nan = __builtin_nanf("");
-  if (j < KVM) {
-    float* dst = p.part_acc + ((row0 + j) * p.splits + split) * D + 4 * g;
+  // ---- the waves of a KV head into one partial (lane (g, j): head j, dims 16nt + 4g + i)
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // lane numbers anew: kept over the loop they cost registers
+  const int tg = (t & 63) >> 4, tj = t & 15;
+  if (tg == 0) {
+    lds_m[w][tj] = m;
+    lds_l[w][tj] = bad ? __builtin_nanf("") : l;
+  }
+  if (tj < KVM) {
+    float* dst = reinterpret_cast<float*>(&lds[w][0]) + tj * OUT_PITCH + 4 * tg;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      *reinterpret_cast<f32x4*>(dst + 16 * nt) = bad ? f32x4{nan, nan, nan, nan} : acc[nt];
-    if (g == 0) {
-      p.part_m[(row0 + j) * p.splits + split] = bad ? nan : m;
-      p.part_l[(row0 + j) * p.splits + split] = bad ? nan : l;
+    for (int nt = 0; nt < NT; ++nt) *reinterpret_cast<f32x4*>(dst + 16 * nt) = acc[nt];
+  }
+  __syncthreads();
+  // From here on a thread holds four dims of one head; where the workgroup has
+  // threads to spare, `teams` of them share the slots that are read back.
+  constexpr int COLS = D / 4, kUnits = KVM * COLS;  // of one KV head
+  static_assert(2 * kUnits <= kThreads, "one unit per thread");
+  const int units = hshift ? 2 * kUnits : kUnits;
+  const int teams = hshift ? kThreads / (2 * kUnits) : kThreads / kUnits;
+  const int team = hshift ? t / (2 * kUnits) : t / kUnits, unit = t - team * units;
+  const int rh = unit / kUnits, rj = unit / COLS - rh * KVM, col = unit % COLS;  // KV head, query head of it, float4 column
+  const int64_t head = ((int64_t)(hg << hshift) + rh) * KVM + rj;
+  Combined c;
+  if (team == 0) {
+    // the waves of KV head rh: rh, rh + hw, ...
+    constexpr int kHalf = kWaves / 2;
+    float mi[kWaves], li[kWaves];
+    f32x4 x[kWaves];
+    auto read = [&](int n) {
+      const int i = rh + (n << hshift);
+      mi[n] = lds_m[i][rj];
+      li[n] = lds_l[i][rj];
+      x[n] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(&lds[i][0]) + rj * OUT_PITCH + 4 * col);
+    };
+    auto fold = [&](int first) {
+      float top = c.m;
+#pragma unroll
+      for (int n = 0; n < kHalf; ++n) top = fmaxf(top, mi[first + n]);
+      c.raise(top);
+#pragma unroll
+      for (int n = 0; n < kHalf; ++n) c.weigh(mi[first + n], li[first + n], x[first + n]);
+    };
+#pragma unroll
+    for (int n = 0; n < kHalf; ++n) read(n);
+    if (!hshift) {
+#pragma unroll
+      for (int n = kHalf; n < kWaves; ++n) read(n);
+      fold(kHalf);
+    }
+    fold(0);
+  }
+  if (slot.k > 1) {
+    // The sequence's partials; offsets from its first slot fit 31 bits.
+    const uint32_t acc_pitch = (uint32_t)q_heads * D * 4, ml_pitch = (uint32_t)q_heads * 8;
+    const __amdgpu_buffer_rsrc_t r_acc = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(part_acc + (int64_t)z0 * q_heads * D), (short)0, (uint32_t)slot.k * acc_pitch, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r_ml = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(part_ml + (int64_t)z0 * q_heads * 2), (short)0, (uint32_t)slot.k * ml_pitch, 0x00020000);
+    const uint32_t acc_at = (uint32_t)head * (D * 4) + 16 * col, ml_at = (uint32_t)head * 8;
+    auto put = [&](int s) {
+      if (team != 0) return;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, c.acc), r_acc, acc_at + s * acc_pitch, 0, kAgent);
+      if (col == 0) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{c.m, c.l}), r_ml, ml_at + s * ml_pitch, 0, kAgent);
+    };
+    // Publishes this workgroup's partial; true in the last of `members`.
+    auto arrive = [&](int z, int members, int level) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partial stores have completed
+      __syncthreads();
+      if (t == 0) lds_last[level] = last_arrival(tickets + (int64_t)z * head_groups + hg, tag, (uint32_t)members);
+      __syncthreads();
+      return __builtin_amdgcn_readfirstlane(lds_last[level]) != 0;
+    };
+    // c = slots s, s + step, ... (`members` of them) combined, eight in flight per thread.
+    auto take = [&](int s, int step, int members) {
+      c = Combined{};
+      if (team < teams) {
+        for (int i0 = team; i0 < members; i0 += 8 * teams) {
+          f32x2 q[8];
+          f32x4 x[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {  // past the end: nothing read, weight 0
+            const int at = i0 + i * teams;
+            const uint32_t from = at < members ? (uint32_t)(s + at * step) : (uint32_t)slot.k;
+            q[i] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r_ml, ml_at + from * ml_pitch, 0, kAgent));
+            x[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r_acc, acc_at + from * acc_pitch, 0, kAgent));
+          }
+          float top = c.m;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            if (i0 + i * teams >= members) q[i][0] = -INFINITY;
+            top = fmaxf(top, q[i][0]);
+          }
+          c.raise(top);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) c.weigh(q[i][0], q[i][1], x[i]);
+        }
+      }
+      if (teams > 1) {
+        f32x4* team_acc = reinterpret_cast<f32x4*>(&lds[0][0]);
+        f32x2* team_ml = reinterpret_cast<f32x2*>(team_acc + kThreads);
+        team_acc[t] = c.acc;
+        team_ml[t] = f32x2{c.m, c.l};
+        __syncthreads();
+        if (team == 0) {
+          float top = c.m;
+          for (int i = 1; i < teams; ++i) top = fmaxf(top, team_ml[t + i * units][0]);
+          c.raise(top);
+          for (int i = 1; i < teams; ++i) {
+            const f32x2 q = team_ml[t + i * units];
+            c.weigh(q[0], q[1], team_acc[t + i * units]);
+          }
+        }
+      }
+    };
+    put(slot.s);
+    if (!arrive(zg, in_group, 0)) return;
+    take(gi * group, 1, in_group);
+    if (groups > 1) {
+      put(gi * group);
+      if (!arrive(z0 + 1, groups, 1)) return;
+      take(0, group, groups);
     }
   }
-}
-
-// Combines the splits as splitkv_paged_mha_fast_stage2_kernel does
-// (paged_mha_fast_kernel.cu:730-799): M = max over splits of m_s,
-// w_s = 2^(m_s - M) for splits with l_s > 0, out = sum_s w_s acc_s / sum_s w_s
-// l_s, and NaN when any split met a bad block id. A row's D/4 float4 columns
-// are shared by `groups` workgroups (gridDim.y), so a step with few rows and
-// hundreds of splits (small batches, long sequences) still spreads over the
-// GPU. In a workgroup, thread t is (split lane t / CPW, column t % CPW): it
-// sums the splits s = lane, lane + LANES, ... of its column, and the lanes'
-// sums meet in an LDS tree.
-constexpr int kCombineThreads = 256;
-
-template <int D>
-__global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(const DecodeParams p) {
-  constexpr int WAVES = kCombineThreads / 64;
-  __shared__ float w_lds[kDecodeMaxSplits];
-  __shared__ float red_m[WAVES], red_s[WAVES];
-  __shared__ int red_nan[WAVES];
-  __shared__ f32x4 part[kCombineThreads];
-  const int t = threadIdx.x, wv = t >> 6, ln = t & 63;
-  const int64_t row = blockIdx.x;
-  const int cpw = (D / 4) / (int)gridDim.y;  // float4 columns of this workgroup
-  const int lanes = kCombineThreads / cpw;
-  const int S = p.splits;
-  const float* m_row = p.part_m + row * S;
-  const float* l_row = p.part_l + row * S;
-  float mx = -INFINITY;
-  int nan = 0;
-  for (int s = t; s < S; s += kCombineThreads) {
-    const float l = l_row[s];
-    nan |= l != l;
-    mx = fmaxf(mx, m_row[s]);
-  }
-  mx = wave_max(mx);
-  const bool wave_nan = __ballot(nan) != 0;
-  if (ln == 0) {
-    red_m[wv] = mx;
-    red_nan[wv] = wave_nan;
-  }
-  __syncthreads();
-  float M = red_m[0];
-  int any_nan = red_nan[0];
+  if (team != 0) return;
+  uint16_t o[4];
 #pragma unroll
-  for (int i = 1; i < WAVES; ++i) {
-    M = fmaxf(M, red_m[i]);
-    any_nan |= red_nan[i];
-  }
-  float den = 0.f;
-  for (int s = t; s < S; s += kCombineThreads) {
-    const float l = l_row[s];
-    const float w = l > 0.f ? exp2f(m_row[s] - M) : 0.f;
-    w_lds[s] = w;
-    den += w > 0.f ? l * w : 0.f;
-  }
-  den = wave_sum(den);
-  if (ln == 0) red_s[wv] = den;
-  __syncthreads();
-  den = red_s[0];
-#pragma unroll
-  for (int i = 1; i < WAVES; ++i) den += red_s[i];
-  // Weighted sum: every split of the row wrote its partial (zeros for an
-  // empty split, whose weight is 0), so the loads need no guard.
-  const int col = (int)blockIdx.y * cpw + t % cpw, lane = t / cpw;
-  const float* acc = p.part_acc + row * S * D + 4 * col;
-  f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = lane; s < S; s += lanes) {
-    const float w = w_lds[s];
-    const f32x4 x = *reinterpret_cast<const f32x4*>(acc + (int64_t)s * D);
-    if (w > 0.f) o += x * w;
-  }
-  part[t] = o;
-  __syncthreads();
-  for (int stride = kCombineThreads / 2; stride >= cpw; stride >>= 1) {
-    if (t < stride) part[t] += part[t + stride];
-    __syncthreads();
-  }
-  if (t < cpw) {
-    const f32x4 sum = part[t];
-    uint16_t* dst = p.out + row * D + 4 * col;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float v = any_nan ? __builtin_nanf("") : (den > 0.f ? sum[e] / den : 0.f);
-      dst[e] = to_bf16(v);
-    }
-  }
-}
-
-// Workgroups per row for the combine: enough to give the GPU ~512
-// workgroups when rows are few (a batch of 64 keeps one per row: splitting
-// its 768 rows measured 4.5 against 4.2 us), at most one per float4 column.
-int combine_groups(int64_t rows, int D) {
-  int g = 1;
-  while (g < D / 4 && rows * g < 512) g *= 2;
-  return g;
-}
-
-// Register sets of one wave. BF16: two. FP8: two (one block in flight)
-// while a split holds at most 48 blocks, four beyond. Both launches on
-// MI355X, FP8, 2 KV heads x 6 query heads, 1 GiB scrub before each step,
-// two sets against four: 64 x 5,040 tokens (16 splits, 20 blocks each)
-// 39.2-39.5 against 41.2-41.3 us; 64 x 10,080 (40 blocks) 68.9 against
-// 72.0; 128 x 5,040 (8 splits, 40 blocks) 68.8-69.2 against 68.0-71.5;
-// 8 x 5,040 (5 blocks) 17.0 against 18.1; 1 x 32,768 (4 blocks) 18.4
-// against 18.9; 64 x 20,160 (79 blocks) 123.2 against 120.7.
-constexpr int kSetsLongSplit = 48;
-
-template <int D, bool kFp8, int KVM, int kSets>
-void launch_sets(const DecodeParams& p, hipStream_t stream, dim3 grid, dim3 block) {
-  if (p.new_k)
-    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, true, kSets>), grid, block, 0, stream, p, p.tables);
-  else
-    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, false, kSets>), grid, block, 0, stream, p, p.tables);
+  for (int e = 0; e < 4; ++e) o[e] = to_bf16(c.l != c.l ? __builtin_nanf("") : (c.l > 0.f ? c.acc[e] / c.l : 0.f));
+  *(gptr<u32x2>)(out + ((int64_t)b * q_heads + head) * D + 4 * col) = u32x2{o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16};
 }
 
 template <int D, bool kFp8, int KVM>
 void launch(const DecodeParams& p, hipStream_t stream) {
-  const int64_t units = (int64_t)p.batch * p.kv_heads * p.splits;
-  const int64_t rows = (int64_t)p.batch * p.q_heads;
-  const dim3 grid((unsigned)((units + kDecodeWaves - 1) / kDecodeWaves)), block(kDecodeWaves * 64);
-  const int per_split = (p.max_blocks + p.splits - 1) / p.splits;
-  if (kFp8 && per_split > kSetsLongSplit) launch_sets<D, kFp8, KVM, 4>(p, stream, grid, block);
-  else launch_sets<D, kFp8, KVM, 2>(p, stream, grid, block);
-  hipLaunchKernelGGL((decode_combine_kernel<D>), dim3((unsigned)rows, (unsigned)combine_groups(rows, D)),
-                     dim3(kCombineThreads), 0, stream, p);
+  const FastDiv by_groups = make_fast_div((uint32_t)(p.kv_heads >> p.hshift));
+  const dim3 grid((unsigned)(p.slots * (p.kv_heads >> p.hshift))), block(kThreads);
+  if (p.new_k)
+    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, true>), grid, block, 0, stream, p.seq_lens, p.tables, p.batch, p.max_blocks, p.slots, p.hshift, by_groups.d, by_groups.mul, by_groups.shift, p);
+  else
+    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, false>), grid, block, 0, stream, p.seq_lens, p.tables, p.batch, p.max_blocks, p.slots, p.hshift, by_groups.d, by_groups.mul, by_groups.shift, p);
 }
 
 template <int D, bool kFp8>
@@ -619,6 +903,47 @@ FastDiv make_fast_div(uint32_t d) {
 uint64_t decode_workspace_bytes(int32_t batch, int32_t q_heads, int32_t head_dim, int32_t splits) {
   const uint64_t rows = (uint64_t)batch * q_heads * splits;
   return rows * head_dim * 4ull + 2ull * rows * 4ull;
+}
+
+namespace {
+// A launch's tag in the arrival tickets: never the same twice in a process,
+// and a word no float, code or id pattern makes (all twelve top bits set).
+uint64_t decode_tag() {
+  static std::atomic<uint64_t> next{std::random_device{}() * 0x9e3779b97f4a7c15ull};
+  return 0xfffull << 41 | (next.fetch_add(1, std::memory_order_relaxed) & ((1ull << 41) - 1));
+}
+}  // namespace
+
+void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes) {
+  const int64_t batch = p->batch;
+  const int row_bytes = p->head_dim * (fp8 ? 1 : 2), chunk = min_chunk(row_bytes);
+  const int64_t most = p->max_blocks <= kWhole ? batch : batch * ((p->max_blocks + chunk - 1) / chunk);  // slots that could hold work
+  // Two KV heads per workgroup read whole 256-byte (FP8) or 512-byte pieces of
+  // a token's row; one per workgroup gives twice the workgroups, which is
+  // better where one per slot would leave the chip idle. MI355X, us: 8 x 5,040
+  // BF16 14.5 against 19.9, 64 mixed up to 300 tokens 11.1 against 12.6; 64
+  // mixed up to 7,040 51.1 (one head) against 41.9.
+  p->hshift = p->kv_heads % 2 == 0 && batch > 16 && most * p->kv_heads > kWorkgroups ? 1 : 0;
+  const int64_t groups = p->kv_heads >> p->hshift;
+  const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 15) & ~(uintptr_t)15;
+  const uint64_t pad = base - reinterpret_cast<uintptr_t>(workspace);
+  const uint64_t slot_bytes = (uint64_t)p->q_heads * (p->head_dim + 2) * 4 + (uint64_t)groups * 8;
+  int64_t slots = (int64_t)((bytes - std::min(bytes, pad)) / slot_bytes);
+  // see find_slot
+  const int64_t one_round = std::max<int64_t>(1, kWorkgroups / groups);
+  const bool twice = batch >= one_round || (row_bytes <= 128 && batch * 8 > one_round);
+  slots = std::min(slots, twice ? 2 * std::max(batch, one_round) : one_round);
+  slots = std::min(slots, most);
+  // One slot per sequence: nothing to combine. Block totals are 32-bit sums,
+  // and a sequence's partials are addressed with 31 bits.
+  if (splits <= 1 || slots <= batch || batch * p->max_blocks > 0x7fffffff ||
+      (int64_t)p->q_heads * p->head_dim * 4 * kDecodeMaxSplits > 0x7fffffff)
+    slots = batch;
+  p->slots = (int32_t)slots;
+  p->tag = decode_tag();
+  p->part_acc = reinterpret_cast<float*>(base);
+  p->part_ml = p->part_acc + (uint64_t)slots * p->q_heads * p->head_dim;
+  p->tickets = reinterpret_cast<uint64_t*>(p->part_ml + (uint64_t)slots * p->q_heads * 2);
 }
 
 hipError_t launch_paged_decode(const DecodeParams& p, bool fp8, hipStream_t stream) {
