@@ -21,14 +21,14 @@ struct ScatterParams {
   uint64_t value_scale_count;
   const int32_t* slots;       // device [tokens], or null: every token takes fixed_slot
   int32_t fixed_slot;
-  uint32_t units;             // tokens * 2 * vecs_per_row (< 2^31)
+  uint32_t units;             // tokens * vecs_per_row (< 2^30)
   uint32_t vecs_per_row;      // row_in_bytes / 16
   uint32_t row_in_bytes;
   uint32_t row_out_bytes;
   uint64_t block_out_bytes;
   uint32_t block_size;
   uint32_t kv_heads;
-  FastDiv by_row_pair;        // 2 * vecs_per_row
+  FastDiv by_row;             // vecs_per_row
   FastDiv by_block_size;
 };
 

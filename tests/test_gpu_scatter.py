@@ -240,3 +240,42 @@ def test_prompt_and_decode_token_written_then_decoded(torch_cuda, fp8):
     got = bf16_to_f64(out.cpu().numpy().view(np.uint16))
     want = O.paged_decode(host, fp8, sc if fp8 else None, layers, heads, head_dim, layer, q, tab, lens)
     assert close(got, want).all()
+
+
+@pytest.mark.parametrize("short", ["key_pool", "value_pool", "key_scales", "value_scales"])
+@pytest.mark.parametrize("f32,fp8", [(False, False), (True, True), (False, True)])
+def test_k_and_v_rows_are_bounded_on_their_own(torch_cuda, short, f32, fp8):
+    """One lane writes a token's K and V vectors: a slot beyond one of the pools
+    (or of the scale pools) still writes the other row, and nothing else."""
+    if not fp8 and short.endswith("scales"):
+        pytest.skip("no scale pools")
+    torch = torch_cuda
+    heads, dim, blocks, n = 3, 64, 12, 77
+    say(f"scatter short {short} f32={f32} fp8={fp8}")
+    rng = np.random.default_rng(5)
+    K, V = _inputs(rng, n, heads, dim, f32)
+    row = heads * dim * (1 if fp8 else 4 if f32 else 2)
+    slots = rng.permutation(blocks * B)[:n].astype(np.int32)
+    # rows (and scales) that each pool admits to have; the short one ends inside a block
+    rows = {k: blocks * B for k in ("key_pool", "value_pool", "key_scales", "value_scales")}
+    rows[short] = 5 * B + 3
+    pool = {k: rng.integers(0, 256, blocks * B * row, dtype=np.uint8) for k in ("key_pool", "value_pool")}
+    scale = {k: np.full(blocks * B * heads, -3.0, np.float32) for k in ("key_scales", "value_scales")}
+    dev = {k: torch.from_numpy(x.copy()).cuda() for k, x in {**pool, **scale}.items()}
+    d_k, d_v = (torch.from_numpy(x.view(np.int16) if not f32 else x).cuda() for x in (K, V))
+    d_slots = torch.from_numpy(slots).cuda()
+    P.scatter_kv(d_k.data_ptr(), d_v.data_ptr(), P.PBE_IN_F32 if f32 else P.PBE_IN_BF16, n, d_slots.data_ptr(), B, heads, dim,
+                 P.PBE_KV_FP8_E4M3 if fp8 else P.PBE_KV_BF16, dev["key_pool"].data_ptr(), rows["key_pool"] * row,
+                 dev["value_pool"].data_ptr(), rows["value_pool"] * row, *((dev["key_scales"].data_ptr(), rows["key_scales"] * heads * 4,
+                 dev["value_scales"].data_ptr(), rows["value_scales"] * heads * 4) if fp8 else (0, 0, 0, 0)), stream=stream_ptr(torch))
+    torch.cuda.synchronize()
+    full_p, full_s = {k: x.copy() for k, x in pool.items()}, {k: x.copy() for k, x in scale.items()}
+    O.scatter_kv(K, V, slots, B, heads, dim, fp8, full_p["key_pool"], full_p["value_pool"], full_s["key_scales"], full_s["value_scales"])
+    for side in ("key", "value"):
+        fits = min(rows[side + "_pool"], rows[side + "_scales"])
+        want, want_s = pool[side + "_pool"].copy(), scale[side + "_scales"].copy()
+        want[: fits * row] = full_p[side + "_pool"][: fits * row]
+        want_s[: fits * heads] = full_s[side + "_scales"][: fits * heads]
+        got = dev[side + "_pool"].cpu().numpy()
+        assert np.array_equal(got, want), (side, first_diff(got, want))
+        assert np.array_equal(dev[side + "_scales"].cpu().numpy(), want_s) or not fp8, side
