@@ -195,12 +195,19 @@ def view_of(ptrs, total_bytes: int, segment_bytes: int | None = None) -> ArenaVi
     return v
 
 
+_AT = (C.c_char * 0).from_buffer
+
+
 def _i32(arr):
     """A contiguous int32 copy (or the array itself) and its address as an int
-    (an int passes to a c_void_p parameter at a fraction of data_as' cost)."""
+    (an int passes to a c_void_p parameter at a fraction of data_as' cost; the
+    buffer's address takes 0.3 us against 1.0 of `ctypes.data`)."""
     import numpy as np
     a = np.ascontiguousarray(arr, dtype=np.int32)
-    return a, a.ctypes.data
+    try:
+        return a, C.addressof(_AT(a))
+    except TypeError:  # a read-only array
+        return a, a.ctypes.data
 
 
 def build_runs(src_ids, dst_ids, kv: KvShape, elem_bytes: int = 2, segment_bytes: int = 0):

@@ -162,3 +162,14 @@ def test_append_reader_rejects_bad_arguments_on_the_host():
         with pytest.raises(P.PbeError) as e:
             P.paged_decode_append(**a)
         assert e.value.code == code, kw
+
+
+@pytest.mark.parametrize("make", [
+    lambda: np.arange(5, dtype=np.int32), lambda: np.arange(5, dtype=np.int64), lambda: [3, 1, 2],
+    lambda: np.arange(24, dtype=np.int32).reshape(4, 6)[:, ::2], lambda: np.zeros(0, np.int32),
+    lambda: np.frombuffer(bytes(12), np.int32),  # read-only
+])
+def test_id_lists_are_passed_by_their_arrays_address(make):
+    a, address = P._i32(make())
+    assert a.dtype == np.int32 and a.flags.c_contiguous
+    assert np.array_equal(a, np.asarray(make(), np.int32)) and address == a.ctypes.data
