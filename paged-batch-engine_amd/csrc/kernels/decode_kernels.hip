@@ -200,11 +200,13 @@ __device__ __forceinline__ int slots_of(int n, uint32_t c) {
 //  - batch < W: W slots. Twice as many (two workgroups per compute unit) read
 //    64 x 5,040 tokens in 65.0 against 57.7 (BF16), 39.2 against 37.8 (FP8):
 //    the second set's slots start and end at the same time as the first's.
-//    But where rows are 128 bytes or less (one workgroup's loads in flight
-//    then do not saturate its compute unit) and W slots would leave a quarter
-//    of the chip idle (160 equal sequences: 160 slots), 2W: FP8 160 x 2,000
-//    tokens 41.4 against 45.7. BF16 rows of 256 bytes gain nothing: 160
-//    mixed up to 1,000 tokens 29.5 against 26.1.
+//    But for FP8, where W slots would leave a quarter of the chip idle (160
+//    equal sequences: 160 slots), 2W: 160 x 2,000 tokens 41.4 against 45.7,
+//    130 x 2,307 44.2 against 50.9. BF16 gains nothing: 130 x 2,307 80.5
+//    against 79.8, 130 x 4,615 of 2 x 64 92.1 against 76.2. (An equal split
+//    count for every sequence took 65 and 71 there: 129 to about 180 equal
+//    BF16 sequences are what the slots do worst, mixed ones of that number
+//    34 against 49 and 56.)
 //  - batch >= W: a sequence is split only where it is longer than 5/4 of the
 //    mean. FP8 256 x 1,000 equal lengths 30.5 against 36.6 with two slots
 //    each, BF16 256 mixed up to 1,000 42.4 against 51.1 with W/2 more slots
@@ -931,7 +933,7 @@ void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspac
   int64_t slots = (int64_t)((bytes - std::min(bytes, pad)) / slot_bytes);
   // see find_slot
   const int64_t one_round = std::max<int64_t>(1, kWorkgroups / groups);
-  const bool twice = batch >= one_round || (row_bytes <= 128 && batch * 8 > one_round);
+  const bool twice = batch >= one_round || (fp8 && batch * 8 > one_round);
   slots = std::min(slots, twice ? 2 * std::max(batch, one_round) : one_round);
   slots = std::min(slots, most);
   // One slot per sequence: nothing to combine. Block totals are 32-bit sums,
