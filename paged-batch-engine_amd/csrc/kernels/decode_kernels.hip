@@ -52,7 +52,7 @@
 // and reading the pages afterwards, byte for byte.
 #include <algorithm>
 #include <atomic>
-#include <random>
+#include <chrono>
 
 #include "decode_kernels.h"
 #include "fp8_device.h"
@@ -909,9 +909,10 @@ uint64_t decode_workspace_bytes(int32_t batch, int32_t q_heads, int32_t head_dim
 
 namespace {
 // A launch's tag in the arrival tickets: never the same twice in a process,
-// and a word no float, code or id pattern makes (all twelve top bits set).
+// and a word no float, code or id pattern makes (all twelve top bits set). The
+// clock keeps processes apart, and unlike a random device it cannot throw.
 uint64_t decode_tag() {
-  static std::atomic<uint64_t> next{std::random_device{}() * 0x9e3779b97f4a7c15ull};
+  static std::atomic<uint64_t> next{(uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() * 0x9e3779b97f4a7c15ull};
   return 0xfffull << 41 | (next.fetch_add(1, std::memory_order_relaxed) & ((1ull << 41) - 1));
 }
 }  // namespace

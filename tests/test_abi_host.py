@@ -173,3 +173,9 @@ def test_id_lists_are_passed_by_their_arrays_address(make):
     a, address = P._i32(make())
     assert a.dtype == np.int32 and a.flags.c_contiguous
     assert np.array_equal(a, np.asarray(make(), np.int32)) and address == a.ctypes.data
+
+
+def test_no_entry_point_can_throw_for_want_of_a_random_device():
+    """std::random_device throws where there is none, and a C entry point must
+    not: the library does not use it."""
+    assert b"random_device" not in P.LIB_PATH.read_bytes()
