@@ -112,10 +112,18 @@ bool accessible(const void* ptr, uint64_t bytes, int device, std::vector<Range>*
   }
   const bool ok_type = (attr.type == hipMemoryTypeDevice && attr.device == device) ||
                        attr.type == hipMemoryTypeHost;
-  const Range r{reinterpret_cast<uint64_t>(base), reinterpret_cast<uint64_t>(base) + size};
+  const Range r{reinterpret_cast<uint64_t>(base), reinterpret_cast<uint64_t>(base) + size,
+                attr.type == hipMemoryTypeHost};
   if (!ok_type || p < r.begin || p + bytes > r.end) return false;
   known->push_back(r);
   return true;
+}
+
+bool on_host(const void* ptr, const std::vector<Range>& known) {
+  const uint64_t p = reinterpret_cast<uint64_t>(ptr);
+  for (const Range& r : known)
+    if (p >= r.begin && p < r.end) return r.host;
+  return false;
 }
 
 bool view_accessible(const pbe_arena_view& v, int device, std::vector<Range>* known) {

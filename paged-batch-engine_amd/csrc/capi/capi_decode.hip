@@ -216,6 +216,7 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   }
   const uint64_t row_bytes = (uint64_t)batch * q_heads * shape->head_dim * 2;
   const uint64_t new_bytes = (uint64_t)batch * shape->kv_heads * shape->head_dim * 2;
+  bool host_workspace = false;
   {
     PBE_DEVICE_SCOPE(device);
     std::vector<Range> known;
@@ -234,6 +235,7 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
         (append && (!accessible(new_keys, new_bytes, device, &known) ||
                     !accessible(new_values, new_bytes, device, &known))))
       return fail(PBE_ERR_INVALID, "decode operands must be memory of device %d", device);
+    host_workspace = !static_scratch && on_host(workspace, known);
   }
   pbe::DecodeParams p{};
   if (pools) {
@@ -274,7 +276,9 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   p.layers = shape->layers;
   p.layer = layer;
   p.max_blocks = max_blocks_per_seq;
-  pbe::plan_decode_slots(&p, fp8, splits, workspace, need);
+  // Arrival tickets are device atomics, which not every link carries to host
+  // memory: with a workspace there every sequence stays whole and takes none.
+  pbe::plan_decode_slots(&p, fp8, host_workspace ? 1 : splits, workspace, need);
   p.half = half;
   p.scale = (1.f / std::sqrt((float)shape->head_dim)) * 1.4426950408889634f;  // as launch_fp8_stage1
   // Largest id whose rows fit: page-major, the whole page (all 2*layers

@@ -61,6 +61,7 @@ bool spans_disjoint(std::vector<std::pair<uint64_t, uint64_t>> dst,
 // ranges are remembered in `known` for the rest of the call.
 struct Range {
   uint64_t begin, end;
+  bool host = false;  // pinned host memory
 };
 
 // Segments of arenas this library created or imported over IPC, per device.
@@ -107,6 +108,8 @@ struct ArenaRegistry {
 ArenaRegistry& arena_registry();
 
 bool accessible(const void* ptr, uint64_t bytes, int device, std::vector<Range>* known);
+// Whether `ptr`, which accessible() has found, lies in pinned host memory.
+bool on_host(const void* ptr, const std::vector<Range>& known);
 bool view_accessible(const pbe_arena_view& v, int device, std::vector<Range>* known);
 
 }  // namespace pbe_capi

@@ -95,3 +95,20 @@ def test_replays_share_a_workspace_with_other_launches(torch_cuda):
         case.run(splits=32, seq_lens=eager)
         assert np.array_equal(got, case.out.cpu().numpy().view(np.uint16)), rep
         assert close(other.run(splits=32, ws=ws), want_other).all(), rep
+
+
+@pytest.mark.parametrize("fp8", [True, False])
+def test_a_workspace_in_pinned_host_memory_takes_no_atomics(torch_cuda, fp8):
+    """Host memory is accepted as a workspace. Arrival tickets there would rest
+    on atomics that the link may not carry (no output, or a wait without end),
+    so nothing of it is touched by them: it keeps its bytes or gets partials."""
+    torch = torch_cuda
+    say(f"decode fp8={fp8}, pinned host workspace")
+    case = DecodeCase(torch, fp8=fp8, layers=1, H=2, D=128, kvm=6, seq_lens=[5000, 31, 0, 2222], seed=22)
+    n = P.decode_workspace_bytes(case.batch, 12, 128, 128)
+    want = case.oracle()
+    for splits in (0, 1, 64):
+        ws = torch.zeros(n, dtype=torch.uint8, pin_memory=True)
+        for _ in range(2):
+            case.out.fill_(7)
+            assert close(case.run(splits=splits, ws=ws), want).all(), splits
