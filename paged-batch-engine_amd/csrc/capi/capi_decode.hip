@@ -276,9 +276,6 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   p.layers = shape->layers;
   p.layer = layer;
   p.max_blocks = max_blocks_per_seq;
-  // Arrival tickets are device atomics, which not every link carries to host
-  // memory: with a workspace there every sequence stays whole and takes none.
-  pbe::plan_decode_slots(&p, fp8, host_workspace ? 1 : splits, workspace, need);
   p.half = half;
   p.scale = (1.f / std::sqrt((float)shape->head_dim)) * 1.4426950408889634f;  // as launch_fp8_stage1
   // Largest id whose rows fit: page-major, the whole page (all 2*layers
@@ -293,7 +290,23 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   p.by_stride = pbe::make_fast_div((uint32_t)stride);
   p.by_seg_pages = pbe::make_fast_div(!pools && kv->nseg > 1 ? (uint32_t)(kv->segment_bytes / page) : 0x7fffffffu);
   PBE_DEVICE_SCOPE(device);
-  PBE_HIP(pbe::launch_paged_decode(p, fp8, static_cast<hipStream_t>(stream)));
+  // A launch takes fewer than 2^32 threads: a batch of more workgroups is read
+  // in parts, one after another on the stream, in the same workspace.
+  const int64_t part = std::max<int64_t>(1, pbe::kDecodeMaxWorkgroups / (2ll * shape->kv_heads));
+  for (int64_t first = 0; first < batch; first += part) {
+    pbe::DecodeParams q = p;
+    q.batch = (int32_t)std::min<int64_t>(part, batch - first);
+    q.seq_lens += first;
+    q.tables += first * max_blocks_per_seq;
+    q.q += first * q_heads * shape->head_dim;
+    q.out += first * q_heads * shape->head_dim;
+    if (append) q.new_k += first * shape->kv_heads * shape->head_dim, q.new_v += first * shape->kv_heads * shape->head_dim;
+    // Arrival tickets are device atomics, which not every link carries to host
+    // memory: with a workspace there every sequence stays whole and takes none.
+    pbe::plan_decode_slots(&q, fp8, host_workspace ? 1 : splits, workspace,
+                           pbe::decode_workspace_bytes(q.batch, q_heads, shape->head_dim, splits));
+    PBE_HIP(pbe::launch_paged_decode(q, fp8, static_cast<hipStream_t>(stream)));
+  }
   return PBE_OK;
 }
 

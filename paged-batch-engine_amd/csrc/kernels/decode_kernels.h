@@ -10,6 +10,9 @@ constexpr int kDecodeMaxSegments = 16;
 constexpr int kDecodeMaxKvMul = 8;    // query heads per KV head held in registers
 constexpr int kDecodeMaxSplits = 1024;  // slots of one sequence
 
+// Of one launch: 2^32 threads less one, in workgroups of 512.
+constexpr int64_t kDecodeMaxWorkgroups = 0xffffffffll / 512;
+
 struct DecodeView {
   const char* base[kDecodeMaxSegments];
   uint64_t segment_bytes;

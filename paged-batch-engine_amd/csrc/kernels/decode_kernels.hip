@@ -136,6 +136,7 @@ struct BlockRegs {
 };
 
 constexpr int kWavesLog = 3, kWaves = 1 << kWavesLog, kThreads = 64 * kWaves;  // of a workgroup
+static_assert(kThreads * kDecodeMaxWorkgroups < (1ll << 32), "a launch has fewer than 2^32 threads");
 // Slots of one sequence that one workgroup combines in one go; more of them
 // are combined in two levels, groups of about the square root first.
 constexpr int kCombineDirect = 64;

@@ -112,3 +112,24 @@ def test_a_workspace_in_pinned_host_memory_takes_no_atomics(torch_cuda, fp8):
         for _ in range(2):
             case.out.fill_(7)
             assert close(case.run(splits=splits, ws=ws), want).all(), splits
+
+
+def test_a_batch_beyond_the_threads_of_one_launch(torch_cuda):
+    """8.5 million sequences of one KV head: more workgroups than a launch
+    takes. The same 128 sequences over and over, so every row is known."""
+    torch = torch_cuda
+    say("decode of 8.5 million sequences")
+    H, D, n, times = 1, 64, 128, 66500
+    small = DecodeCase(torch, fp8=True, layers=1, H=H, D=D, kvm=1, seq_lens=[1 + i % 40 for i in range(n)], seed=23)
+    want = small.run(splits=1)
+    assert close(want, small.oracle()).all()
+    want = small.out.clone()
+    batch = n * times
+    q, tables, lens = (x.repeat(times, *([1] * (x.dim() - 1))) for x in (small.q, small.t_dev, small.s_dev))
+    out = torch.zeros_like(q)
+    ws = torch.empty(P.decode_workspace_bytes(batch, 1, D, 1), dtype=torch.uint8, device="cuda")
+    P.paged_decode(small.view, P.PBE_KV_FP8_E4M3, small.scales.data_ptr(), small.scales.numel() * 4, small.kv, small.layer, q.data_ptr(),
+                   out.data_ptr(), batch, 1, tables.data_ptr(), lens.data_ptr(), small.max_blocks, 1, ws.data_ptr(), ws.numel(),
+                   stream_ptr(torch))
+    torch.cuda.synchronize()
+    assert bool((out.view(times, n, -1) == want.view(1, n, -1)).all())
