@@ -119,6 +119,31 @@ bool accessible(const void* ptr, uint64_t bytes, int device, std::vector<Range>*
   return true;
 }
 
+int64_t compute_units(int device) {
+  static std::mutex mu;
+  static int cus[64] = {};
+  if (device < 0 || device >= 64) return 256;
+  std::lock_guard<std::mutex> lock(mu);
+  if (!cus[device]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) {
+      (void)hipGetLastError();
+      n = 256;
+    }
+    cus[device] = n;
+  }
+  return cus[device];
+}
+
+int64_t compute_units() {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  return compute_units(device);
+}
+
 bool on_host(const void* ptr, const std::vector<Range>& known) {
   const uint64_t p = reinterpret_cast<uint64_t>(ptr);
   for (const Range& r : known)

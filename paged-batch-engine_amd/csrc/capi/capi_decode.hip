@@ -19,30 +19,6 @@
 using namespace pbe_capi;
 
 
-namespace {
-// Compute units of the calling thread's current GPU (256 on MI355X), cached
-// per device; 256 when the runtime cannot say.
-int64_t decode_cus() {
-  static std::mutex mu;
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  std::lock_guard<std::mutex> lock(mu);
-  if (!cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-}  // namespace
-
 extern "C" {
 
 int32_t pbe_paged_decode_splits(int32_t batch, int32_t kv_heads, int32_t max_blocks_per_seq,
@@ -53,7 +29,7 @@ int32_t pbe_paged_decode_splits(int32_t batch, int32_t kv_heads, int32_t max_blo
   // (decode_kernels.hip). One wave per SIMD (4 per CU) of the current GPU,
   // rounded down; FP8 pages take two per SIMD when every split still holds at
   // least 8 blocks; at least 4 blocks (64 tokens) per split.
-  const int64_t simds = 4ll * decode_cus();
+  const int64_t simds = 4ll * compute_units();
   const int64_t units = (int64_t)batch * kv_heads;
   int64_t splits = std::max<int64_t>(1, simds / units);
   if (kv_dtype == PBE_KV_FP8_E4M3) {
@@ -290,6 +266,7 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   p.by_stride = pbe::make_fast_div((uint32_t)stride);
   p.by_seg_pages = pbe::make_fast_div(!pools && kv->nseg > 1 ? (uint32_t)(kv->segment_bytes / page) : 0x7fffffffu);
   PBE_DEVICE_SCOPE(device);
+  p.workgroups = (int32_t)compute_units(device);
   // A launch takes fewer than 2^32 threads: a batch of more workgroups is read
   // in parts, one after another on the stream, in the same workspace.
   const int64_t part = std::max<int64_t>(1, pbe::kDecodeMaxWorkgroups / (2ll * shape->kv_heads));

@@ -108,6 +108,10 @@ struct ArenaRegistry {
 ArenaRegistry& arena_registry();
 
 bool accessible(const void* ptr, uint64_t bytes, int device, std::vector<Range>* known);
+// Compute units of a GPU (256 on MI355X), cached; 256 when the runtime cannot
+// say. Without an argument: of the calling thread's current GPU.
+int64_t compute_units(int device);
+int64_t compute_units();
 // Whether `ptr`, which accessible() has found, lies in pinned host memory.
 bool on_host(const void* ptr, const std::vector<Range>& known);
 bool view_accessible(const pbe_arena_view& v, int device, std::vector<Range>* known);

@@ -40,6 +40,8 @@ struct DecodeParams {
   float* part_ml;          // [slots][q_heads][2]: maximum, sum
   uint64_t* tickets;       // [slots][kv_heads >> hshift]
   uint64_t tag;            // of this launch (decode_tag())
+  int32_t workgroups;      // that fill the GPU: one per compute unit
+  int32_t one_round;       // slots that are one workgroup per compute unit
   int32_t slots;           // >= batch; == batch: one slot per sequence, no partials
   int32_t hshift;          // log2 of the KV heads read by one workgroup
   int32_t batch, q_heads, kv_heads, head_dim, layers, layer, max_blocks;

@@ -140,7 +140,6 @@ static_assert(kThreads * kDecodeMaxWorkgroups < (1ll << 32), "a launch has fewer
 // Slots of one sequence that one workgroup combines in one go; more of them
 // are combined in two levels, groups of about the square root first.
 constexpr int kCombineDirect = 64;
-constexpr int kWorkgroups = 256;  // one per compute unit
 // A sequence of at most kWhole blocks stays whole; a longer one is cut into
 // slots of at least min_chunk blocks (a row: one token of one KV head). us:
 // 64 mixed up to 19 blocks, BF16 x 128, 9.8 whole against 11.0; 10 x 47 blocks
@@ -196,8 +195,8 @@ __device__ __forceinline__ int slots_of(int n, uint32_t c) {
 // scan over the batch. (A binary search in every wave took 3.6 us of a batch
 // of 160, 10 us with two workgroups per compute unit; this takes 1.6 and 3.)
 //
-// How many slots (W = kWorkgroups / workgroups per slot = one per compute
-// unit; us on MI355X, 2 KV heads x 128 unless said otherwise):
+// How many slots (W = the GPU's compute units / workgroups per slot; us on
+// MI355X, 256 of them, 2 KV heads x 128 unless said otherwise):
 //  - batch < W: W slots. Twice as many (two workgroups per compute unit) read
 //    64 x 5,040 tokens in 65.0 against 57.7 (BF16), 39.2 against 37.8 (FP8):
 //    the second set's slots start and end at the same time as the first's.
@@ -416,7 +415,7 @@ __global__ __launch_bounds__(kThreads, 4) void paged_decode_kernel(
   const int head_groups = (int)groups_d, kv_heads = head_groups << hshift;
   const int z = (int)fast_div(blockIdx.x, FastDiv{groups_d, groups_mul, groups_shift});
   const int hg = (int)blockIdx.x - z * head_groups;
-  const Slot slot = find_slot<min_chunk(D * E)>(fit, lens, batch, max_blocks, slots, max(1, kWorkgroups / head_groups), z, w, lane);
+  const Slot slot = find_slot<min_chunk(D * E)>(fit, lens, batch, max_blocks, slots, p.one_round, z, w, lane);
   if (slot.b < 0) return;
   const int b = slot.b, seq = slot.seq;
   // Of the workgroup's waves, every (1 << hshift)th reads the same KV head:
@@ -927,14 +926,15 @@ void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspac
   // better where one per slot would leave the chip idle. MI355X, us: 8 x 5,040
   // BF16 14.5 against 19.9, 64 mixed up to 300 tokens 11.1 against 12.6; 64
   // mixed up to 7,040 51.1 (one head) against 41.9.
-  p->hshift = p->kv_heads % 2 == 0 && batch > 16 && most * p->kv_heads > kWorkgroups ? 1 : 0;
+  p->hshift = p->kv_heads % 2 == 0 && batch > 16 && most * p->kv_heads > p->workgroups ? 1 : 0;
   const int64_t groups = p->kv_heads >> p->hshift;
   const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 15) & ~(uintptr_t)15;
   const uint64_t pad = base - reinterpret_cast<uintptr_t>(workspace);
   const uint64_t slot_bytes = (uint64_t)p->q_heads * (p->head_dim + 2) * 4 + (uint64_t)groups * 8;
   int64_t slots = (int64_t)((bytes - std::min(bytes, pad)) / slot_bytes);
   // see find_slot
-  const int64_t one_round = std::max<int64_t>(1, kWorkgroups / groups);
+  const int64_t one_round = std::max<int64_t>(1, p->workgroups / groups);
+  p->one_round = (int32_t)one_round;
   const bool twice = batch >= one_round || (fp8 && batch * 8 > one_round);
   slots = std::min(slots, twice ? 2 * std::max(batch, one_round) : one_round);
   slots = std::min(slots, most);
