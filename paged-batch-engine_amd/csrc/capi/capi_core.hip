@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -120,19 +121,16 @@ bool accessible(const void* ptr, uint64_t bytes, int device, std::vector<Range>*
 }
 
 int64_t compute_units(int device) {
-  static std::mutex mu;
-  static int cus[64] = {};
+  static std::atomic<int> cus[64] = {};
   if (device < 0 || device >= 64) return 256;
-  std::lock_guard<std::mutex> lock(mu);
-  if (!cus[device]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cus[device] = n;
+  int n = cus[device].load(std::memory_order_relaxed);
+  if (n) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) {
+    (void)hipGetLastError();
+    n = 256;
   }
-  return cus[device];
+  cus[device].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 int64_t compute_units() {

@@ -80,14 +80,15 @@ int scatter_call(const void* keys, const void* values, int32_t in_dtype, int32_t
   p.value_scale_count = fp8 ? value_scale_bytes / 4 : 0;
   p.slots = slots;
   p.fixed_slot = fixed_slot;
-  p.units = (uint32_t)(units / 2);  // one lane moves a vector of K and the same of V
+  p.pairs = pbe::scatter_pairs(units / 2, fp8, compute_units(device));
+  p.units = (uint32_t)(p.pairs ? units / 2 : units);
   p.vecs_per_row = (uint32_t)(row_in / 16);
   p.row_in_bytes = (uint32_t)row_in;
   p.row_out_bytes = (uint32_t)row_out;
   p.block_out_bytes = (uint64_t)block_size * row_out;
   p.block_size = (uint32_t)block_size;
   p.kv_heads = (uint32_t)kv_heads;
-  p.by_row = pbe::make_fast_div(p.vecs_per_row);
+  p.by_row = pbe::make_fast_div(p.pairs ? p.vecs_per_row : 2 * p.vecs_per_row);
   p.by_block_size = pbe::make_fast_div((uint32_t)block_size);
   PBE_DEVICE_SCOPE(device);
   PBE_HIP(pbe::launch_scatter_kv(p, f32, fp8, lanes, static_cast<hipStream_t>(stream)));

@@ -279,3 +279,37 @@ def test_k_and_v_rows_are_bounded_on_their_own(torch_cuda, short, f32, fp8):
         got = dev[side + "_pool"].cpu().numpy()
         assert np.array_equal(got, want), (side, first_diff(got, want))
         assert np.array_equal(dev[side + "_scales"].cpu().numpy(), want_s) or not fp8, side
+
+
+# K and V vectors of all tokens, in workgroups of 256: one lane takes one of them
+# up to 512 workgroups (of FP8 pages; others from 257 on), a pair beyond.
+@pytest.mark.parametrize("f32,fp8", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("workgroups", [1, 256, 257, 512, 513])
+def test_both_sides_of_the_pairs_rule(torch_cuda, workgroups, f32, fp8):
+    torch = torch_cuda
+    heads, dim = 3, 64
+    vectors = heads * dim * (4 if f32 else 2) // 16
+    n = workgroups * 256 // vectors  # the last token that fits the workgroups
+    assert (n * vectors + 255) // 256 == workgroups and ((n + 11) * vectors + 255) // 256 > workgroups
+    say(f"scatter {n} tokens, {workgroups} workgroups, f32={f32} fp8={fp8}")
+    rng = np.random.default_rng(workgroups)
+    K, V = _inputs(rng, n, heads, dim, f32)
+    blocks = n // B + 2
+    slots = rng.permutation(blocks * B)[:n].astype(np.int32)
+    slots[n // 3] = -1
+    e = 1 if fp8 else 4 if f32 else 2
+    pool = [rng.integers(0, 256, blocks * B * heads * dim * e, dtype=np.uint8) for _ in range(2)]
+    scale = [np.full(blocks * B * heads, -3.0, np.float32) for _ in range(2)]
+    d_pool, d_scale = ([torch.from_numpy(x.copy()).cuda() for x in y] for y in (pool, scale))
+    d_k, d_v = (torch.from_numpy(x.view(np.int16) if not f32 else x).cuda() for x in (K, V))
+    d_slots = torch.from_numpy(slots).cuda()
+    sc = [x for d in d_scale for x in (d.data_ptr(), d.numel() * 4)] if fp8 else [0, 0, 0, 0]
+    P.scatter_kv(d_k.data_ptr(), d_v.data_ptr(), P.PBE_IN_F32 if f32 else P.PBE_IN_BF16, n, d_slots.data_ptr(), B, heads, dim,
+                 P.PBE_KV_FP8_E4M3 if fp8 else P.PBE_KV_BF16, *[x for d in d_pool for x in (d.data_ptr(), d.numel())], *sc,
+                 stream=stream_ptr(torch))
+    torch.cuda.synchronize()
+    O.scatter_kv(K, V, slots, B, heads, dim, fp8, *pool, *scale)
+    for got, want in zip(d_pool, pool):
+        assert np.array_equal(got.cpu().numpy(), want), first_diff(got.cpu().numpy(), want)
+    for got, want in zip(d_scale, scale):
+        assert not fp8 or np.array_equal(got.cpu().numpy(), want)
