@@ -917,16 +917,33 @@ uint64_t decode_tag() {
 }
 }  // namespace
 
+namespace {
+// Two KV heads per workgroup read whole 256-byte (FP8) or 512-byte pieces of
+// a token's row; one per workgroup gives twice the workgroups, which is
+// better where one per slot would leave the chip idle. MI355X, us: 8 x 5,040
+// BF16 14.5 against 19.9, 64 mixed up to 300 tokens 11.1 against 12.6; 64
+// mixed up to 7,040 51.1 (one head) against 41.9. In small batches it needs
+// more blocks per workgroup the fewer of a token's bytes lie beside the
+// head's: 4 x 128 BF16 16 x 9,000 55.9 against 61.8 (mixed 33.0 against 35.4),
+// 8 x 4,000 mixed 17.1 against 15.3; FP8 16 x 9,000 36.7 against 40.1, 8 x
+// 16,000 mixed 24.3 against 23.2; 8 x 128 8 x 4,000 FP8 24.3 against 28.2; 2 x
+// 64 FP8 16 x 9,000 18.7 against 22.5.
+bool head_pairs(const DecodeParams& p, bool fp8, int64_t most) {
+  if (p.kv_heads % 2 || most * p.kv_heads <= p.workgroups) return false;
+  if (p.batch > 16) return true;
+  const int64_t each = (int64_t)p.batch * p.max_blocks * p.kv_heads / p.workgroups;  // blocks of one head per workgroup
+  if (p.head_dim * (fp8 ? 1 : 2) == 64 && p.kv_heads < 8) return p.batch >= 4 && each >= 64;
+  if (p.kv_heads >= 8) return each >= (fp8 ? 20 : p.batch <= 8 ? 16 : 36);
+  if (p.kv_heads >= 4) return each >= (p.batch >= 12 ? (fp8 ? 48 : 32) : p.batch >= 6 ? (fp8 ? 192 : 64) : fp8 ? INT32_MAX : 120);
+  return p.head_dim == 128 && !fp8 && p.batch >= 12 && each >= 110;
+}
+}  // namespace
+
 void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes) {
   const int64_t batch = p->batch;
   const int row_bytes = p->head_dim * (fp8 ? 1 : 2), chunk = min_chunk(row_bytes);
   const int64_t most = p->max_blocks <= kWhole ? batch : batch * ((p->max_blocks + chunk - 1) / chunk);  // slots that could hold work
-  // Two KV heads per workgroup read whole 256-byte (FP8) or 512-byte pieces of
-  // a token's row; one per workgroup gives twice the workgroups, which is
-  // better where one per slot would leave the chip idle. MI355X, us: 8 x 5,040
-  // BF16 14.5 against 19.9, 64 mixed up to 300 tokens 11.1 against 12.6; 64
-  // mixed up to 7,040 51.1 (one head) against 41.9.
-  p->hshift = p->kv_heads % 2 == 0 && batch > 16 && most * p->kv_heads > p->workgroups ? 1 : 0;
+  p->hshift = head_pairs(*p, fp8, most) ? 1 : 0;
   const int64_t groups = p->kv_heads >> p->hshift;
   const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 15) & ~(uintptr_t)15;
   const uint64_t pad = base - reinterpret_cast<uintptr_t>(workspace);

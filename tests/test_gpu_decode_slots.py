@@ -133,3 +133,15 @@ def test_a_batch_beyond_the_threads_of_one_launch(torch_cuda):
                    stream_ptr(torch))
     torch.cuda.synchronize()
     assert bool((out.view(times, n, -1) == want.view(1, n, -1)).all())
+
+
+@pytest.mark.parametrize("fp8,H,D,kvm,lens", [
+    (False, 4, 128, 2, [300] * 5 + [2000, 8210, 0]),      # 514 table columns x 8 x 4: over 64 blocks of a head per workgroup
+    (False, 4, 128, 7, [600] * 13 + [2500]),              # over 32, a batch of 12 or more
+    (True, 8, 64, 1, [1300] * 9),                         # 8 heads, FP8: over 20
+    (True, 2, 64, 7, [200] * 7 + [16600]),               # 64-byte rows: over 64
+])
+def test_small_batches_of_paired_heads(torch_cuda, fp8, H, D, kvm, lens):
+    say(f"decode paired heads, a batch of {len(lens)}: fp8={fp8} H{H} D{D} kvm{kvm}")
+    case = DecodeCase(torch_cuda, fp8=fp8, layers=1, H=H, D=D, kvm=kvm, seq_lens=lens, seed=24)
+    assert close(case.run(), case.oracle()).all()
