@@ -68,6 +68,7 @@ ABI_HOST_SOURCES = [
 HIP_SOURCES = [
     "csrc/kernels/handoff_kernels.hip",
     "csrc/kernels/decode_kernels.hip",
+    "csrc/kernels/decode_split_kernels.hip",
     "csrc/kernels/scatter_kernels.hip",
     "csrc/capi/capi_core.hip",
     "csrc/capi/capi_arena.hip",
@@ -78,6 +79,7 @@ HIP_SOURCES = [
 ]
 CPU_TESTS = ["tests/cpp/test_drop_in_api.cpp"]
 GPU_TESTS = ["tests/cpp/test_gpu_backend.cpp"]
+DECODE_PLAN = "tests/cpp/decode_plan.cpp"  # host code: prints how the decode reader would read a batch
 
 
 def _run(cmd: list[str]) -> None:
@@ -125,6 +127,8 @@ def build(jobs: int = 8) -> Path:
     # tests can replay identical scenarios on it and on the reference build.
     _run(["g++", *CXX_FLAGS, "-shared", *INCLUDES, str(ROOT / "oracle" / "ref_driver.cpp"), *cpu_objs,
           "-o", str(LIB / "libpbe_api_driver.so")])
+    _run([HIPCC, "-x", "c++", "-D__HIP_PLATFORM_AMD__", *CXX_FLAGS, *INCLUDES, "-I/opt/rocm/include", str(ROOT / DECODE_PLAN),
+          f"-L{LIB}", "-lpbe_handoff", "-Wl,-rpath,$ORIGIN", "-o", str(LIB / "pbe_decode_plan")])
     for t in GPU_TESTS:
         _run([HIPCC, *HIP_FLAGS, *INCLUDES, f"-I{ROOT / 'tests' / 'cpp'}", str(ROOT / t),
               f"-L{LIB}", "-lpbe_handoff", "-Wl,-rpath,$ORIGIN",

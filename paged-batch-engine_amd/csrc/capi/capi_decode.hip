@@ -269,7 +269,7 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
   p.workgroups = (int32_t)compute_units(device);
   // A launch takes fewer than 2^32 threads: a batch of more workgroups is read
   // in parts, one after another on the stream, in the same workspace.
-  const int64_t part = std::max<int64_t>(1, pbe::kDecodeMaxWorkgroups / (2ll * shape->kv_heads));
+  const int64_t part = std::max<int64_t>(1, pbe::kDecodeMaxWorkgroups / (host_workspace ? (int64_t)q_heads * splits : 2ll * shape->kv_heads));
   for (int64_t first = 0; first < batch; first += part) {
     pbe::DecodeParams q = p;
     q.batch = (int32_t)std::min<int64_t>(part, batch - first);
@@ -278,10 +278,9 @@ int paged_decode_call(const pbe_arena_view* kv, int32_t kv_dtype, const float* s
     q.q += first * q_heads * shape->head_dim;
     q.out += first * q_heads * shape->head_dim;
     if (append) q.new_k += first * shape->kv_heads * shape->head_dim, q.new_v += first * shape->kv_heads * shape->head_dim;
-    // Arrival tickets are device atomics, which not every link carries to host
-    // memory: with a workspace there every sequence stays whole and takes none.
-    pbe::plan_decode_slots(&q, fp8, host_workspace ? 1 : splits, workspace,
-                           pbe::decode_workspace_bytes(q.batch, q_heads, shape->head_dim, splits));
+    // Arrival tickets are device atomics, which not every link carries to host memory.
+    pbe::plan_decode_slots(&q, fp8, splits, workspace, pbe::decode_workspace_bytes(q.batch, q_heads, shape->head_dim, splits),
+                           !host_workspace);
     PBE_HIP(pbe::launch_paged_decode(q, fp8, static_cast<hipStream_t>(stream)));
   }
   return PBE_OK;

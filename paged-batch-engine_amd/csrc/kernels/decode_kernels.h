@@ -26,6 +26,12 @@ struct FastDiv {
 };
 FastDiv make_fast_div(uint32_t d);
 
+// How a batch is read: in slots by one launch (decode_kernels.hip), in equal
+// splits by two (decode_split_kernels.hip), or in splits if its sequences are
+// of about equal length and in slots otherwise. Lengths are device memory, so
+// for the last all three kernels are launched and look at them.
+enum class DecodeMode : int32_t { kSlots, kSplits, kEither };
+
 struct DecodeParams {
   DecodeView kv;           // payload arena (FP8: int8 E4M3 planes; BF16: bf16 planes)
   const float* scales;     // FP8 only: page-major [layer][K|V][token][kv_head] fp32
@@ -42,6 +48,12 @@ struct DecodeParams {
   uint64_t tag;            // of this launch (decode_tag())
   int32_t workgroups;      // that fill the GPU: one per compute unit
   int32_t one_round;       // slots that are one workgroup per compute unit
+  DecodeMode mode;
+  // Splits: partial results of one per (sequence, query head, split).
+  int32_t splits;
+  float* split_acc;        // [batch][q_heads][splits][head_dim]
+  float* split_m;          // [batch][q_heads][splits]
+  float* split_l;          // [batch][q_heads][splits]
   int32_t slots;           // >= batch; == batch: one slot per sequence, no partials
   int32_t hshift;          // log2 of the KV heads read by one workgroup
   int32_t batch, q_heads, kv_heads, head_dim, layers, layer, max_blocks;
@@ -66,10 +78,12 @@ struct DecodeParams {
 // Bytes of a workspace that holds the partials of `splits` slots per sequence.
 uint64_t decode_workspace_bytes(int32_t batch, int32_t q_heads, int32_t head_dim, int32_t splits);
 
-// Lays the slots out in `bytes` bytes at `workspace` (at least
-// decode_workspace_bytes(.., splits) of them) and sets p.part_acc .. p.hshift.
-void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes);
+// Lays slots and splits out in `bytes` bytes at `workspace` (at least
+// decode_workspace_bytes(.., splits) of them) and sets p.one_round .. p.hshift.
+// `atomics`: whether the workspace takes device atomics, which the slots need.
+void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes, bool atomics);
 
 hipError_t launch_paged_decode(const DecodeParams& p, bool fp8, hipStream_t stream);
+hipError_t launch_paged_decode_splits(const DecodeParams& p, bool fp8, hipStream_t stream);
 
 }  // namespace pbe

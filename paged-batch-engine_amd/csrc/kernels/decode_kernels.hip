@@ -35,13 +35,14 @@
 //    slot order, so the result does not depend on which one that is.
 //
 // What bounds it: large batches the HBM rate (64 sequences of 5,040 tokens,
-// 2 KV heads x 128: FP8 36.8 us, 4.6 TB/s over the call; the loop alone reads
-// at 6.3), small ones the chain of dependent reads (arguments, lengths, block
-// table, rows, partials, ticket, partials: 1 x 5,040 tokens, 2 x 64 BF16,
-// 10.6 us). Two launches with an equal split count for every sequence took,
-// in the same order, 37.8 and 11.0; 64 sequences of mixed lengths up to 7,040
-// BF16 62.1 (now 40.5); a layer of 8 mixed up to 16,384, 4 x 128 FP8, 30.2
-// (21.3).
+// 2 KV heads x 128: FP8 36.3 us, 4.7 TB/s over the call), small ones the chain
+// of dependent reads (arguments, lengths, block table, rows, partials, ticket,
+// partials: 4 x 5,040 tokens, 2 x 64 BF16, 11.4 us). Two launches with an equal
+// split count for every sequence take, in the same order, 37.5 and 11.1; 64
+// sequences of mixed lengths up to 7,040 BF16 62.0 (here 40.2); a layer of 8
+// mixed up to 16,384, 4 x 128 FP8, 29.0 (21.2). They remain in
+// decode_split_kernels.hip for the calls they are the faster at: see
+// decode_mode().
 //
 // Append variant (kAppend): the step's new token of every sequence, at its
 // last position, is written into its page slot by the one wave that reads
@@ -54,86 +55,12 @@
 #include <atomic>
 #include <chrono>
 
-#include "decode_kernels.h"
-#include "fp8_device.h"
+#include "decode_device.h"
 
 namespace pbe {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-using gptr = __attribute__((address_space(1))) T*;  // global memory
-
-constexpr int kBlockTokens = 16;
 constexpr int kStream = 0x02;  // buffer load policy: non-temporal
-
-template <int kCtrl>
-__device__ __forceinline__ float dpp(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xf, 0xf, false));
-}
-
-// Max / sum over the four lanes j, j+16, j+32, j+48 with the gfx950 row
-// swaps (VALU only, no LDS round trip). Every lane ends with the same value,
-// combined in the same order.
-__device__ __forceinline__ float group_max4(float x) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
-__device__ __forceinline__ float group_sum4(float x) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
-// Orders this wave's LDS writes before its other lanes' reads.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// fp32 -> bf16, round to nearest even; NaN stays NaN (quiet).
-__device__ __forceinline__ uint16_t to_bf16(float f) {
-  const uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-  return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
-
-__device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv& f) {
-  return (__umulhi(n, f.mul) + n) >> f.shift;
-}
-
-// Four E4M3 bytes -> four BF16 with the gfx950 scaled converter (scale 1: exact).
-__device__ __forceinline__ u32x2 e4m3x4_to_bf16x4_cvt(uint32_t w) {
-  return u32x2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w, 1.0f, false)),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)w, 1.0f, true))};
-}
-
-// Per-lane registers of one block of 16 tokens of one KV head: the lane's
-// part of key row j, its whole-row-mapped part of the value tile and one scale.
-template <int D, bool kFp8>
-struct Geo {
-  static constexpr int E = kFp8 ? 1 : 2;
-  static constexpr int WORDS = D * E / 16;   // key words = value words per lane
-  static constexpr int PITCH = D * E + 16;   // LDS row pitch of the value tile
-};
-
-template <int W, bool kFp8>
-struct BlockRegs {
-  uint32_t k[W];
-  uint32_t v[W];
-  // FP8: lane (g, n): log2(e)/sqrt(D) * key scale (n%8 < 4) or value scale
-  // (otherwise) of token 4g + n%4
-  float scale;
-};
 
 constexpr int kWavesLog = 3, kWaves = 1 << kWavesLog, kThreads = 64 * kWaves;  // of a workgroup
 static_assert(kThreads * kDecodeMaxWorkgroups < (1ll << 32), "a launch has fewer than 2^32 threads");
@@ -163,24 +90,6 @@ __device__ __forceinline__ int wave_scan(int x) {
   return scan_step<0x143, 0xc>(x);  // row_bcast 31 into rows 2 and 3
 }
 __device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
-template <int kCtrl>
-__device__ __forceinline__ int max_step(int x) {
-  return max(x, __builtin_amdgcn_update_dpp(x, x, kCtrl, 0xf, 0xf, false));
-}
-__device__ __forceinline__ int wave_max_int(int x) {
-  x = max_step<0xb1>(x);
-  x = max_step<0x4e>(x);
-  x = max_step<0x141>(x);
-  x = max_step<0x140>(x);
-  return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
-             max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
-}
-
-// Blocks of a length; a bad one (negative, or beyond the table) has none.
-__device__ __forceinline__ int blocks_of(int seq, int max_blocks) {
-  const int n = seq > 0 ? (int)(((uint32_t)seq + kBlockTokens - 1) / kBlockTokens) : 0;
-  return n <= max_blocks ? n : 0;
-}
 // Slots of a sequence of n blocks at c blocks per slot.
 __device__ __forceinline__ int slots_of(int n, uint32_t c) {
   return n <= kWhole ? 1 : (int)(((uint32_t)n + c - 1) / c);
@@ -188,8 +97,8 @@ __device__ __forceinline__ int slots_of(int n, uint32_t c) {
 
 // One slot: a chunk of one sequence's blocks. The chunk length c is the same
 // for the whole batch, so a batch of mixed lengths keeps every workgroup
-// equally busy: a sequence of n blocks takes max(1, ceil(n / c)) slots, c
-// being about the shortest (at least min_chunk) whose slots fit the slots of
+// equally busy: a sequence of n blocks takes ceil(n / c) slots (one if n is at
+// most kWhole), c being about the shortest (at least min_chunk) whose slots fit the slots of
 // the launch. The lengths are device memory, so each workgroup works this out
 // for itself: its waves try one c each, then find their slot with a prefix
 // scan over the batch. (A binary search in every wave took 3.6 us of a batch
@@ -203,10 +112,9 @@ __device__ __forceinline__ int slots_of(int n, uint32_t c) {
 //    But for FP8, where W slots would leave a quarter of the chip idle (160
 //    equal sequences: 160 slots), 2W: 160 x 2,000 tokens 41.4 against 45.7,
 //    130 x 2,307 44.2 against 50.9. BF16 gains nothing: 130 x 2,307 80.5
-//    against 79.8, 130 x 4,615 of 2 x 64 92.1 against 76.2. (An equal split
-//    count for every sequence took 65 and 71 there: 129 to about 180 equal
-//    BF16 sequences are what the slots do worst, mixed ones of that number
-//    34 against 49 and 56.)
+//    against 79.8, 130 x 4,615 of 2 x 64 92.1 against 76.2. Equal lengths that
+//    leave W slots idle are read in splits instead (decode_mode()); mixed ones
+//    of that number take 34 against 49 and 56 here.
 //  - batch >= W: a sequence is split only where it is longer than 5/4 of the
 //    mean. FP8 256 x 1,000 equal lengths 30.5 against 36.6 with two slots
 //    each, BF16 256 mixed up to 1,000 42.4 against 51.1 with W/2 more slots
@@ -365,7 +273,7 @@ struct Combined {
 template <int D, bool kFp8, int KVM, bool kAppend>
 __global__ __launch_bounds__(kThreads, 4) void paged_decode_kernel(
     const int32_t* __restrict__ lens, const int32_t* __restrict__ tables, const int batch, const int max_blocks, const int slots,
-    const int hshift, const uint32_t groups_d, const uint32_t groups_mul, const uint32_t groups_shift,
+    const int hshift_mode, const uint32_t groups_d, const uint32_t groups_mul, const uint32_t groups_shift,
     const DecodeParams p) {
   using G = Geo<D, kFp8>;
   constexpr int E = G::E;
@@ -384,7 +292,8 @@ __global__ __launch_bounds__(kThreads, 4) void paged_decode_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char lds_new[kAppend ? kWaves : 1][kAppend ? 2 * D * E : 16];
   __shared__ bf16x8 lds_q[kWaves][NK][64];
 
-  // The arguments that follow the preloaded ones, read in one go: left to
+  const int hshift = hshift_mode & 0xff;
+  // The arguments that follow the first ones, read in one go: left to
   // itself the compiler reads each where it is used, one scalar round trip
   // after another.
   gptr<const char> kv0 = (gptr<const char>)p.kv.base[0];
@@ -412,6 +321,7 @@ __global__ __launch_bounds__(kThreads, 4) void paged_decode_kernel(
   }
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((hshift_mode >> 8) == (int)DecodeMode::kEither && alike(lens, batch, max_blocks, lane)) return;
   const int head_groups = (int)groups_d, kv_heads = head_groups << hshift;
   const int z = (int)fast_div(blockIdx.x, FastDiv{groups_d, groups_mul, groups_shift});
   const int hg = (int)blockIdx.x - z * head_groups;
@@ -870,9 +780,9 @@ void launch(const DecodeParams& p, hipStream_t stream) {
   const FastDiv by_groups = make_fast_div((uint32_t)(p.kv_heads >> p.hshift));
   const dim3 grid((unsigned)(p.slots * (p.kv_heads >> p.hshift))), block(kThreads);
   if (p.new_k)
-    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, true>), grid, block, 0, stream, p.seq_lens, p.tables, p.batch, p.max_blocks, p.slots, p.hshift, by_groups.d, by_groups.mul, by_groups.shift, p);
+    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, true>), grid, block, 0, stream, p.seq_lens, p.tables, p.batch, p.max_blocks, p.slots, p.hshift | (int)p.mode << 8, by_groups.d, by_groups.mul, by_groups.shift, p);
   else
-    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, false>), grid, block, 0, stream, p.seq_lens, p.tables, p.batch, p.max_blocks, p.slots, p.hshift, by_groups.d, by_groups.mul, by_groups.shift, p);
+    hipLaunchKernelGGL((paged_decode_kernel<D, kFp8, KVM, false>), grid, block, 0, stream, p.seq_lens, p.tables, p.batch, p.max_blocks, p.slots, p.hshift | (int)p.mode << 8, by_groups.d, by_groups.mul, by_groups.shift, p);
 }
 
 template <int D, bool kFp8>
@@ -918,6 +828,55 @@ uint64_t decode_tag() {
 }  // namespace
 
 namespace {
+// How the batch is read; `slots` of one_round are one workgroup per compute
+// unit. us on MI355X, the whole call, two launches against one:
+//  - Few sequences: one launch combines a sequence's slots in one workgroup per
+//    KV head, the second launch in up to 32. 1 x 16,384 tokens 2 x 128 BF16
+//    14.2 and 17.2, 1 x 9,000 12.9 and 15.7, 2 x 5,040 12.9 and 13.9, 4 x 2,000
+//    of 8 x 128 FP8 12.7 and 14.0; up to 160 blocks of less than 8 x 128 the
+//    other way round, 2 x 2,000 12.4 and 11.7.
+//  - Small batches of 64-dim heads, where finding the slot counts: 16 x 1,000
+//    tokens 2 x 64 10.7 and 11.3, 8 x 2,000 10.9 and 11.3; 4 x 5,040 11.1 and
+//    11.4, mixed 11.0 and 10.8.
+//  - 64-byte rows that head_pairs() cannot or does not join: 32 x 4,000 of 5 x
+//    64 32.3 and 41.6 (mixed 25.7 and 27.9), of 3 x 64 23.9 and 30.9 (20.1 and
+//    20.0), 16 x 4,000 of 16 x 64 47.3 and 57.8 (42.8 and 48.0).
+//  - Equal lengths whose whole slots leave compute units idle: 130 x 2,000 2 x
+//    128 BF16 55 and 70, 153 x 2,000 62 and 80, 65 x 4,500 of 4 x 128 117 and
+//    167, FP8 66 and 80; or of many or an odd number of KV heads, whose rows
+//    the two launches read whole: 48 x 4,000 of 8 x 128 FP8 92 and 106, 64 x
+//    3,000 of 5 x 128 57 and 75. Mixed lengths are the reverse (130 mixed up to
+//    7,000 131 and 36), so there the kernels look at them; the launches that
+//    find nothing to do cost about 3 us.
+DecodeMode decode_mode(const DecodeParams& p, bool fp8, int32_t splits, int64_t one_round, bool atomics) {
+  if (splits <= 1) return DecodeMode::kSlots;
+  if (!atomics) return DecodeMode::kSplits;
+  if (p.max_blocks <= kWhole) return DecodeMode::kSlots;
+  const int64_t batch = p.batch, blocks = batch * p.max_blocks, rows = blocks * p.kv_heads;
+  const bool odd = p.kv_heads % 2 && p.kv_heads >= 3;
+  const bool few = batch <= 2 || batch * p.kv_heads <= 3;
+  if (p.kv_heads >= 8 ? few || rows <= 4096 : p.head_dim == 64 ? few || blocks <= 1100 : few && p.max_blocks > 160) return DecodeMode::kSplits;
+  const int64_t out_rows = batch * p.q_heads;  // each costs the combining launch a workgroup
+  if (fp8 && p.head_dim == 64 && (odd || p.kv_heads >= 16) && out_rows * splits <= 1 << 26) return DecodeMode::kSplits;
+  if (odd && rows >= 100ll * p.workgroups && batch < 2 * one_round && out_rows <= 2048) return DecodeMode::kEither;
+  if (batch >= one_round || out_rows > 3072) return DecodeMode::kSlots;
+  if (rows >= 64ll * p.workgroups) {
+    // Of the launch's slots those that equal lengths would use, in percent. The
+    // line, at 2,000 tokens each, two launches, one, and both as they look at
+    // the lengths: BF16 2 x 128 87 (two slots each, 67%) 38.4, 42.2, 41.5; 66
+    // (three, 77%) 30.6, 32.4, 33.5; 179 (one, 70%, and no more than two splits)
+    // 82, 79; 2 x 64 130 (51%) 36.3, 41.4, 39.4, 168 (66%) 37.1, 38.6. FP8 4 x
+    // 128 65 (three, 76%) 36.4, 42.6, 39.6; 89 (two, 70%) 47, 56, 50.7; 96 (75%)
+    // 48.5, 49.2, 52.3.
+    const int64_t used = fp8 ? 2 * one_round : one_round, each = used / batch, full = 100 * each * batch / used;
+    const bool idle = p.head_dim == 64 ? !fp8 && each == 1 && full < 66
+                      : fp8            ? full < (each == 3 ? 78 : 72) && each <= 3
+                                       : full < 79 && each <= 2 && splits >= each + 2;
+    if (idle) return DecodeMode::kEither;
+  }
+  return p.kv_heads >= 8 && rows >= 180ll * p.workgroups ? DecodeMode::kEither : DecodeMode::kSlots;
+}
+
 // Two KV heads per workgroup read whole 256-byte (FP8) or 512-byte pieces of
 // a token's row; one per workgroup gives twice the workgroups, which is
 // better where one per slot would leave the chip idle. MI355X, us: 8 x 5,040
@@ -939,7 +898,7 @@ bool head_pairs(const DecodeParams& p, bool fp8, int64_t most) {
 }
 }  // namespace
 
-void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes) {
+void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspace, uint64_t bytes, bool atomics) {
   const int64_t batch = p->batch;
   const int row_bytes = p->head_dim * (fp8 ? 1 : 2), chunk = min_chunk(row_bytes);
   const int64_t most = p->max_blocks <= kWhole ? batch : batch * ((p->max_blocks + chunk - 1) / chunk);  // slots that could hold work
@@ -952,6 +911,7 @@ void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspac
   // see find_slot
   const int64_t one_round = std::max<int64_t>(1, p->workgroups / groups);
   p->one_round = (int32_t)one_round;
+  p->mode = decode_mode(*p, fp8, splits, one_round, atomics);
   const bool twice = batch >= one_round || (fp8 && batch * 8 > one_round);
   slots = std::min(slots, twice ? 2 * std::max(batch, one_round) : one_round);
   slots = std::min(slots, most);
@@ -965,9 +925,17 @@ void plan_decode_slots(DecodeParams* p, bool fp8, int32_t splits, void* workspac
   p->part_acc = reinterpret_cast<float*>(base);
   p->part_ml = p->part_acc + (uint64_t)slots * p->q_heads * p->head_dim;
   p->tickets = reinterpret_cast<uint64_t*>(p->part_ml + (uint64_t)slots * p->q_heads * 2);
+  p->splits = splits;
+  p->split_acc = static_cast<float*>(workspace);
+  p->split_m = p->split_acc + (uint64_t)batch * p->q_heads * splits * p->head_dim;
+  p->split_l = p->split_m + (uint64_t)batch * p->q_heads * splits;
 }
 
 hipError_t launch_paged_decode(const DecodeParams& p, bool fp8, hipStream_t stream) {
+  if (p.mode != DecodeMode::kSlots) {
+    const hipError_t e = launch_paged_decode_splits(p, fp8, stream);
+    if (e != hipSuccess || p.mode == DecodeMode::kSplits) return e;
+  }
   bool ok = false;
   if (p.head_dim == 128) ok = fp8 ? launch_kvm<128, true>(p, stream) : launch_kvm<128, false>(p, stream);
   else if (p.head_dim == 64) ok = fp8 ? launch_kvm<64, true>(p, stream) : launch_kvm<64, false>(p, stream);

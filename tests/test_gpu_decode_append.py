@@ -356,3 +356,23 @@ def test_arena_form_on_a_segmented_arena(torch_cuda, fp8):
     want_out = O.paged_decode(want, fp8, want_sc, layers, H, D, layer, case.q_host, case.tables,
                               case.seq_lens)
     assert close(bf16_to_f64(fused), want_out).all()
+
+
+@pytest.mark.parametrize("fp8,H,D,kvm,lens,splits", [
+    (False, 2, 128, 6, [16 * 8 * 64 + 1, 5, 300], 0),              # 65 slots: two levels of combining
+    (True, 2, 64, 7, [16 * 16 * 64 + 1, 5, 300], 0),
+    (False, 2, 128, 2, [16 * 64 * 8, 16 * 64 * 8 + 1, 9001], 1),   # the last block at and past a wave's 64 block ids
+    (True, 2, 128, 2, [16 * 64 * 4 + 1, 4700] + [9] * 18, 1),      # two KV heads per workgroup
+    (False, 2, 128, 1, [1010 - i % 30 for i in range(130)], 0),    # about equal lengths: splits
+    (False, 2, 128, 1, [1010 - 7 * i for i in range(130)], 0),     # the same batch, mixed: slots
+    (True, 4, 128, 1, [1020] * 65, 0),
+])
+def test_append_over_every_way_to_read_a_batch(torch_cuda, fp8, H, D, kvm, lens, splits):
+    say(f"decode append fp8={fp8} H={H} D={D} kvm={kvm} {len(lens)} sequences up to {max(lens)} splits={splits}")
+    step = Step(torch_cuda, fp8, H, D, kvm, lens, seed=31)
+    a, b = step.two_step(splits), step.fused(splits)
+    _same(a, b)
+    pools = _oracle_pools(step)
+    assert np.array_equal(b["kp"], pools[0]) and np.array_equal(b["vp"], pools[1])
+    want = O.paged_decode_pools(b["kp"], b["vp"], fp8, b.get("ks"), b.get("vs"), H, D, step.q, step.tables, lens)
+    assert close(bf16_to_f64(b["out"]), want).all()
