@@ -304,11 +304,23 @@ int pbe_copy_ops(const pbe_copy_op* ops, int64_t n_ops, int device, void* stream
  * outside the arena or not a page id, or whose length needs more than
  * max_blocks_per_seq blocks, gets NaN outputs (its pages are not read past
  * the failing id). splits = 0 picks pbe_paged_decode_splits(); at most 1024.
- * `splits` sizes the partials: the batch's blocks are cut into pieces of about
- * equal length, at most batch * splits of them (longer sequences take more
- * than `splits`, shorter ones fewer); 1 leaves every sequence whole.
+ * `splits` sizes the partials. A batch is read by one launch, its blocks cut
+ * into pieces of about equal length, at most batch * splits of them (longer
+ * sequences take more than `splits`, shorter ones fewer), or by two launches,
+ * every sequence cut into `splits` equal pieces, whichever is faster for the
+ * shape (where that depends on the lengths, the kernels look at them). 1 leaves
+ * every sequence whole. So the order of a sequence's sums, and with it the last
+ * bits of its output, depends on the batch it is in and on `splits`, not on
+ * `splits` alone; for one batch they are the same on every call. A batch of
+ * mixed lengths with more sequences than the GPU has compute units gains from
+ * splits of 2 or more, which pbe_paged_decode_splits() does not pick for BF16.
  * workspace: at least pbe_paged_decode_workspace_bytes() bytes of device
- * memory, used by this launch until it completes. Asynchronous on `stream`. */
+ * memory, used by this launch until it completes; it may hold anything when the
+ * launch starts. It takes 64-bit device atomics; in pinned host memory, which
+ * is accepted, none are used and the reading is slower. A captured call keeps
+ * its marks in it: no other work may write the workspace while a replay runs,
+ * and one that was disturbed that way needs it cleared before the next replay.
+ * Asynchronous on `stream`. */
 #define PBE_KV_BF16 0
 #define PBE_KV_FP8_E4M3 1
 /* Split count for a decode launch on the current GPU (its CU count sets the
@@ -334,8 +346,9 @@ int pbe_paged_decode(const pbe_arena_view* kv, int32_t kv_dtype, const float* sc
  * capture, tight serving loops, harnesses that forbid hipMalloc). The split-K
  * partials live in a static device array of PBE_DECODE_SCRATCH_BYTES per GPU
  * (held until the process ends) instead of a caller workspace; nothing is
- * allocated and nothing in it needs clearing. splits = 0 takes pbe_paged_decode_splits' count, lowered until the
- * partials fit the array; an explicit split count whose partials need more
+ * allocated and nothing in it needs clearing. splits = 0 takes
+ * pbe_paged_decode_splits' count, lowered until the partials fit the array; an
+ * explicit split count whose partials need more
  * (pbe_paged_decode_workspace_bytes) is rejected with PBE_ERR_INVALID, as is a
  * batch too large for the array even at one split. All calls on
  * one GPU share the array, so calls must not overlap in time: issue them on

@@ -118,7 +118,10 @@ __device__ __forceinline__ int slots_of(int n, uint32_t c) {
 //  - batch >= W: a sequence is split only where it is longer than 5/4 of the
 //    mean. FP8 256 x 1,000 equal lengths 30.5 against 36.6 with two slots
 //    each, BF16 256 mixed up to 1,000 42.4 against 51.1 with W/2 more slots
-//    than sequences.
+//    than sequences. With the automatic split count BF16 has the slots for it
+//    up to batch = W with two KV heads per workgroup, FP8 up to 2W; beyond, that
+//    count is 1 and every sequence stays whole (mixed up to 7,000, 2 x 128 BF16:
+//    256 86, 257 191; two launches 202 and 293) unless the caller asks for 2.
 struct Slot {
   int b = -1;  // sequence; -1: no work for this workgroup
   int seq = 0;
