@@ -5,6 +5,7 @@ Compiles, in-tree:
                           drop-in API (include/{base,cache,serving}/*.h)
   lib/pbe_cpp_tests       C++ unit tests of the drop-in API (host-only parts)
   lib/pbe_cpp_gpu_tests   C++ tests that need a GPU (HIP backend, connector)
+  lib/pbe_decode_plan     prints how the decode reader would read a batch (tests)
   lib/libpbe_ceiling.so   measurement-only read/write stream kernels (bench.py)
 
 Usage: python paged-batch-engine_amd/build.py [--jobs N]

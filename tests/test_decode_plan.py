@@ -38,7 +38,7 @@ def auto(batch, kv, group, dim, fp8, blocks, cus=256, atomics=1, address=4096):
     ((87, 2, 6, 128, 0, 125), EITHER), ((66, 2, 6, 128, 0, 125), SLOTS), ((65, 4, 7, 128, 0, 125), EITHER), ((65, 4, 7, 128, 1, 125), EITHER),
     ((96, 4, 7, 128, 1, 125), SLOTS), ((89, 4, 7, 128, 1, 125), EITHER), ((130, 2, 7, 64, 0, 125), EITHER), ((130, 2, 7, 64, 1, 125), SLOTS),
     ((48, 8, 4, 128, 1, 250), EITHER), ((130, 2, 6, 128, 0, 30), SLOTS),  # short ones have nothing to win
-    # the listed kinds of work of large batches stay with one launch
+    # large and mixed batches: one launch
     ((64, 2, 6, 128, 1, 315), SLOTS), ((64, 2, 6, 128, 0, 440), SLOTS), ((8, 4, 7, 128, 1, 1024), SLOTS), ((256, 2, 6, 128, 0, 440), SLOTS),
 ])
 def test_how_a_batch_is_read(case, mode):
